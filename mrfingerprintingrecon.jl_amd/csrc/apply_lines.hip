@@ -2,8 +2,9 @@
 // ext/MRISubspaceReconCUDAExt/NFFTNormalOp.jl:193-218 for every grid the line
 // FFTs cover (each 2N 2,3,5-smooth up to 2048) and any number of coefficients
 // K, in 2D and 3D.  The fused passes (apply2d*.hip, apply3d*.hip) cover the
-// common shapes (2N in the fused length set, up to 512, K <= 8) faster; this
-// path takes the rest.
+// common shapes (2N in the fused length set, up to 512, K <= 8) faster, the
+// fused line passes (planes.hip) every other one with K <= 8 and rows up to
+// 1024; this path takes the rest.
 //
 // For a chunk of Cb coils at a time, with the grids of the chunk in two
 // ping-pong buffers A and B of Cb K prod(2N) elements:
@@ -142,12 +143,6 @@ int lines_chunk_coils(const msr_normalop* op) {
     return (int)std::min<int64_t>(cb, op->C);
 }
 
-size_t lines_scratch_bytes(const msr_normalop* op, size_t es) {
-    int64_t g = (int64_t)op->Cb * op->K;
-    for (int a = 0; a < op->d; ++a) g *= 2 * op->N[a];
-    return es * (size_t)g;
-}
-
 template <class AT>
 static void lines_passes_t(msr_normalop* op, const AT* b, int c_begin, int c_end, hipStream_t st,
                            const int* skip) {
@@ -160,8 +155,8 @@ static void lines_passes_t(msr_normalop* op, const AT* b, int c_begin, int c_end
     AT* bufA = op->T.as<AT>();
     AT* bufB = op->T2.as<AT>();
     AT* partial = op->partial.as<AT>();
-    MSR_REQUIRE(op->T.bytes >= lines_scratch_bytes(op, sizeof(AT)) &&
-                    op->T2.bytes >= lines_scratch_bytes(op, sizeof(AT)),
+    MSR_REQUIRE(op->T.bytes >= sizeof(AT) * general_scratch(op, 0) &&
+                    op->T2.bytes >= sizeof(AT) * general_scratch(op, 1),
                 MSR_ERR_ERROR, "apply scratch not allocated for this precision");
     auto line = [&](int nf, int dir, int lin, int lout) {
         LinePass p;

@@ -171,11 +171,29 @@ __device__ __forceinline__ void cart_accumulate(double2 (&acc)[K * (K + 1) / 2],
         }
 }
 
+// Where the kernel keeps entry e = j + K k of cell q: along the last image axis
+// (lam[(line P + e) n + i], the order the fused line passes read) or cell by
+// cell (lam[q P + e]).
+struct CartLam {
+    int64_t lines, n;  // cells q = line + lines * i with i < n; lines = 0: cell by cell
+    int P;
+    __device__ __forceinline__ int64_t operator()(int64_t q, int e) const {
+        if (!lines) return q * P + e;
+        const int64_t i = q / lines;
+        return ((q - i * lines) * P + e) * n + i;
+    }
+};
+
+static CartLam cart_lam(const msr_normalop* op) {
+    const int64_t n = op->N[op->d - 1];
+    return {op->planes ? op->V / n : 0, n, op->P};
+}
+
 // Writes the full K x K block of cell q (lower triangle = conjugate) and its
 // kmask flag: Λ[1,1] != 0 after rounding to the kernel's element type.
 template <int K, bool REAL>
 __device__ __forceinline__ void cart_store(const double2 (&acc)[K * (K + 1) / 2], int64_t q,
-                                           void* lam, uint8_t* flag) {
+                                           CartLam at, void* lam, uint8_t* flag) {
     const bool keep = REAL ? ((float)acc[0].x != 0.f)
                            : ((float)acc[0].x != 0.f || (float)acc[0].y != 0.f);
     flag[q] = keep ? 1 : 0;
@@ -185,7 +203,7 @@ __device__ __forceinline__ void cart_store(const double2 (&acc)[K * (K + 1) / 2]
 #pragma unroll
         for (int j = 0; j <= k; ++j, ++p) {
             const double2 v = keep ? acc[p] : make_double2(0.0, 0.0);
-            const int64_t o1 = q * K * K + j + K * k, o2 = q * K * K + k + K * j;
+            const int64_t o1 = at(q, j + K * k), o2 = at(q, k + K * j);
             if (REAL) {
                 static_cast<float*>(lam)[o1] = (float)v.x;
                 static_cast<float*>(lam)[o2] = (float)v.x;
@@ -202,7 +220,8 @@ __global__ __launch_bounds__(256) void cart_kernel_traj(const int* __restrict__ 
                                                         const int* __restrict__ offs,
                                                         const int* __restrict__ frame,
                                                         const void* __restrict__ U, int64_t nt,
-                                                        int64_t G, void* __restrict__ lam,
+                                                        int64_t G, CartLam at,
+                                                        void* __restrict__ lam,
                                                         uint8_t* __restrict__ flag) {
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < G;
          q += (int64_t)gridDim.x * blockDim.x) {
@@ -211,7 +230,7 @@ __global__ __launch_bounds__(256) void cart_kernel_traj(const int* __restrict__ 
         for (int p = 0; p < K * (K + 1) / 2; ++p) acc[p] = make_double2(0.0, 0.0);
         for (int e = offs[q]; e < offs[q + 1]; ++e)
             cart_accumulate<K, REAL>(acc, U, frame[perm[e]], nt, 1.0);
-        cart_store<K, REAL>(acc, q, lam, flag);
+        cart_store<K, REAL>(acc, q, at, lam, flag);
     }
 }
 
@@ -220,7 +239,8 @@ __global__ __launch_bounds__(256) void cart_kernel_traj(const int* __restrict__ 
 template <int K, bool REAL>
 __global__ __launch_bounds__(256) void cart_kernel_mask(const uint8_t* __restrict__ M, CartN g,
                                                         int64_t nt, const void* __restrict__ U,
-                                                        int64_t G, void* __restrict__ lam,
+                                                        int64_t G, CartLam at,
+                                                        void* __restrict__ lam,
                                                         uint8_t* __restrict__ flag) {
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < G;
          q += (int64_t)gridDim.x * blockDim.x) {
@@ -236,14 +256,14 @@ __global__ __launch_bounds__(256) void cart_kernel_mask(const uint8_t* __restric
         for (int p = 0; p < K * (K + 1) / 2; ++p) acc[p] = make_double2(0.0, 0.0);
         for (int64_t t = 0; t < nt; ++t)
             if (M[src + t * G]) cart_accumulate<K, REAL>(acc, U, t, nt, 1.0);
-        cart_store<K, REAL>(acc, q, lam, flag);
+        cart_store<K, REAL>(acc, q, at, lam, flag);
     }
 }
 
 // FFTNormalOp(Λ) (src/FFTNormalOp.jl:38-47): the given (K, K, N...) kernel,
 // zero on the cells off kmask = Λ[1,1] != 0 (kept in full, as the reference).
 template <class LT>
-__global__ void cart_kernel_dense(const LT* __restrict__ in, int KK, int64_t G,
+__global__ void cart_kernel_dense(const LT* __restrict__ in, int KK, int64_t G, CartLam at,
                                   LT* __restrict__ lam, uint8_t* __restrict__ flag) {
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < G * KK;
          e += (int64_t)gridDim.x * blockDim.x) {
@@ -253,7 +273,7 @@ __global__ void cart_kernel_dense(const LT* __restrict__ in, int KK, int64_t G,
         if constexpr (sizeof(LT) == sizeof(float)) keep = l11 != 0.f;
         else keep = l11.x != 0.f || l11.y != 0.f;
         if (e == q * KK) flag[q] = keep ? 1 : 0;
-        lam[e] = keep ? in[e] : LT{};
+        lam[at(q, (int)(e - q * KK))] = keep ? in[e] : LT{};
     }
 }
 
@@ -320,11 +340,11 @@ void cart_build_kernel(msr_normalop* op, const msr_traj* traj, const uint8_t* M,
         if (u_real)                                                                              \
             hipLaunchKernelGGL((cart_kernel_traj<KK, true>), dim3(grid), dim3(256), 0, st,       \
                                plan.perm.as<int>(), plan.offs.as<int>(), traj->frame.as<int>(), \
-                               U, traj->nt, G, op->lam->p, flag.as<uint8_t>());                  \
+                               U, traj->nt, G, cart_lam(op), op->lam->p, flag.as<uint8_t>());                  \
         else                                                                                     \
             hipLaunchKernelGGL((cart_kernel_traj<KK, false>), dim3(grid), dim3(256), 0, st,      \
                                plan.perm.as<int>(), plan.offs.as<int>(), traj->frame.as<int>(), \
-                               U, traj->nt, G, op->lam->p, flag.as<uint8_t>());                  \
+                               U, traj->nt, G, cart_lam(op), op->lam->p, flag.as<uint8_t>());                  \
     }
         MSR_CART_K(MSR_CART_T)
 #undef MSR_CART_T
@@ -333,10 +353,10 @@ void cart_build_kernel(msr_normalop* op, const msr_traj* traj, const uint8_t* M,
     if (K == KK) {                                                                              \
         if (u_real)                                                                             \
             hipLaunchKernelGGL((cart_kernel_mask<KK, true>), dim3(grid), dim3(256), 0, st, M, g, \
-                               nt_mask, U, G, op->lam->p, flag.as<uint8_t>());                  \
+                               nt_mask, U, G, cart_lam(op), op->lam->p, flag.as<uint8_t>());                  \
         else                                                                                    \
             hipLaunchKernelGGL((cart_kernel_mask<KK, false>), dim3(grid), dim3(256), 0, st, M,  \
-                               g, nt_mask, U, G, op->lam->p, flag.as<uint8_t>());               \
+                               g, nt_mask, U, G, cart_lam(op), op->lam->p, flag.as<uint8_t>());               \
     }
         MSR_CART_K(MSR_CART_M)
 #undef MSR_CART_M
@@ -355,11 +375,11 @@ void cart_load_dense(msr_normalop* op, const void* lambda, hipStream_t st) {
     const int grid = (int)std::min<int64_t>((G * KK + 255) / 256, 16384);
     if (op->lam_real)
         hipLaunchKernelGGL(cart_kernel_dense<float>, dim3(grid), dim3(256), 0, st,
-                           static_cast<const float*>(lambda), KK, G, op->lam->as<float>(),
+                           static_cast<const float*>(lambda), KK, G, cart_lam(op), op->lam->as<float>(),
                            flag.as<uint8_t>());
     else
         hipLaunchKernelGGL(cart_kernel_dense<float2>, dim3(grid), dim3(256), 0, st,
-                           static_cast<const float2*>(lambda), KK, G, op->lam->as<float2>(),
+                           static_cast<const float2*>(lambda), KK, G, cart_lam(op), op->lam->as<float2>(),
                            flag.as<uint8_t>());
     MSR_CHECK_LAUNCH();
     cart_kmask(op, flag.as<uint8_t>(), G, st);

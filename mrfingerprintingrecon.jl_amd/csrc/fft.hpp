@@ -398,6 +398,39 @@ constexpr bool fft_plan_exact() {
     return true;
 }
 
+// v[r] *= W_{NS R}^{k r} for the stage with radix R after the product NS of the
+// earlier radices (stage-ordered table: entry NS - R0 + (r - 1) NS + k).
+template <int N, int R, int NS, int DIR, class CT>
+__device__ __forceinline__ void stage_twiddle(CT* v, const CT* tw, int k) {
+    if constexpr (NS > 1) {
+        constexpr int OFF = NS - FFTPlan<N>::R[0];
+        if constexpr (sizeof(CT) == 16 && R == 8) {
+            // ComplexF64: two table twiddles, the others by products
+            // (rounding <= 3 ulp), fewer LDS reads and registers
+            CT w1 = tw[OFF + k], w4 = tw[OFF + 3 * NS + k];
+            if constexpr (DIR > 0) {
+                w1.y = -w1.y;
+                w4.y = -w4.y;
+            }
+            const CT w2 = cmul(w1, w1), w3 = cmul(w2, w1);
+            v[1] = cmul(v[1], w1);
+            v[2] = cmul(v[2], w2);
+            v[3] = cmul(v[3], w3);
+            v[4] = cmul(v[4], w4);
+            v[5] = cmul(v[5], cmul(w4, w1));
+            v[6] = cmul(v[6], cmul(w4, w2));
+            v[7] = cmul(v[7], cmul(w4, w3));
+        } else {
+#pragma unroll
+            for (int r = 1; r < R; ++r) {
+                CT w = tw[OFF + (r - 1) * NS + k];
+                if constexpr (DIR > 0) w.y = -w.y;
+                v[r] = cmul(v[r], w);
+            }
+        }
+    }
+}
+
 // One stage.  MODE bit 0: the inputs come from reg (reg[p R + r] = x[j + r N/R]
 // for j = t + p T) instead of LDS; bit 1: the outputs go to reg (for the last
 // stage reg[p R + r] = X[j + r N/R]) instead of LDS.
@@ -428,34 +461,7 @@ __device__ __forceinline__ void fft_stage(CT* buf, const CT* tw, int t, bool act
         const int j = t + p * T;
         if (active && (EXACT || j < NB)) {
             const int k = j % NS;
-            if constexpr (NS > 1) {
-                // stage-ordered table: W_{NS R}^{k r} at OFF + (r - 1) NS + k
-                constexpr int OFF = NS - FFTPlan<N>::R[0];
-                if constexpr (sizeof(CT) == 16 && R == 8) {
-                    // ComplexF64: two table twiddles, the others by products
-                    // (rounding <= 3 ulp), fewer LDS reads and registers
-                    CT w1 = tw[OFF + k], w4 = tw[OFF + 3 * NS + k];
-                    if constexpr (DIR > 0) {
-                        w1.y = -w1.y;
-                        w4.y = -w4.y;
-                    }
-                    const CT w2 = cmul(w1, w1), w3 = cmul(w2, w1);
-                    v[p][1] = cmul(v[p][1], w1);
-                    v[p][2] = cmul(v[p][2], w2);
-                    v[p][3] = cmul(v[p][3], w3);
-                    v[p][4] = cmul(v[p][4], w4);
-                    v[p][5] = cmul(v[p][5], cmul(w4, w1));
-                    v[p][6] = cmul(v[p][6], cmul(w4, w2));
-                    v[p][7] = cmul(v[p][7], cmul(w4, w3));
-                } else {
-#pragma unroll
-                    for (int r = 1; r < R; ++r) {
-                        CT w = tw[OFF + (r - 1) * NS + k];
-                        if constexpr (DIR > 0) w.y = -w.y;
-                        v[p][r] = cmul(v[p][r], w);
-                    }
-                }
-            }
+            stage_twiddle<N, R, NS, DIR>(v[p], tw, k);
             Butterfly<R, DIR>::run(v[p]);
             const int base = (j - k) * R + k;
 #pragma unroll

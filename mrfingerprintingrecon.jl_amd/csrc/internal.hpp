@@ -160,6 +160,8 @@ struct msr_normalop {
     int G = 1, Gb = 1;                // coil groups of pass C / of pass B (3D)
     msr::ApplyKnobs knobs[3];         // fused 2D launch choices per apply mode
     bool fused = true;                // fused Toeplitz passes (else the line-kernel apply)
+    bool planes = false;              // the others: fused line passes (planes.hpp), and the
+                                      // Cartesian kernel stored along them
     int Cb = 1;                       // coils per chunk of the line-kernel apply
     // CG state (allocated on first use)
     msr::DevBuf cg_r, cg_u, cg_c, cg_scal, cg_part, cg_x64, cg_u32;

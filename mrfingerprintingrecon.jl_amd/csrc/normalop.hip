@@ -16,6 +16,7 @@
 #include "apply3d.hpp"
 #include "fft.hpp"
 #include "normalop.hpp"
+#include "planes.hpp"
 
 namespace msr {
 
@@ -109,10 +110,14 @@ void remember_knobs(const msr_normalop* op, int am, const ApplyKnobs& k) {
 void op_alloc_scratch(msr_normalop* op) {
     const int64_t ny = op->N[1];
     op->Cb = 1;
-    if (!op->cart && !op->fused) {
+    if (op->cart || !op->fused) {
+        op->Cb = op->cart ? op->C : lines_chunk_coils(op);
+        // coil groups of the three-pass 2D apply: enough workgroups (of four rows
+        // or more) for the combine to fill the chip, about four per CU
         op->G = 1;
+        if (op->planes && op->d == 2)
+            op->G = (int)std::max<int64_t>(1, std::min<int64_t>(op->Cb, 1024 / (ceil_div(ny, 4) * op->K)));
         op->Gb = 1;
-        op->Cb = lines_chunk_coils(op);
     } else if (op->d == 2 && !op->cart) {
         const int tiles = tiles2d((int)ny, 8);
         int G = (int)ceil_div(512, (int64_t)tiles * op->K);
@@ -139,6 +144,18 @@ void op_alloc_scratch(msr_normalop* op) {
     op_ensure_scratch(op, false);
 }
 
+// Elements of T (which = 0) and T2 (1) of the applies outside the fused
+// Toeplitz passes, for Cb coils at a time: the fused line passes keep the
+// zero-padded last axis in LDS (T2 only in 3D); the separate line passes
+// ping-pong two whole grids.
+size_t general_scratch(const msr_normalop* op, int which) {
+    const int pad = op->cart ? 1 : 2;
+    int64_t g = (int64_t)op->Cb * op->K * pad * op->N[0];
+    if (!op->planes) return (size_t)(g * pad * op->N[1] * (op->d == 3 ? pad * op->N[2] : 1));
+    if (op->d == 2) return which ? 0 : (size_t)(g * op->N[1]);
+    return (size_t)(g * op->N[2] * op->N[1] * (which ? pad : 1));
+}
+
 // Intermediates for the apply precision (grow-only: ComplexF64 needs twice the
 // bytes).  Re-allocation changes the addresses, which the graph keys include.
 void op_ensure_scratch(msr_normalop* op, bool f64) {
@@ -152,12 +169,9 @@ void op_ensure_scratch(msr_normalop* op, bool f64) {
     const size_t es = f64 ? sizeof(double2) : sizeof(float2);
     if (op->scratch_es >= es) return;
     const int64_t nx = op->N[0], ny = op->N[1], nz = op->N[2];
-    if (op->cart) {  // two ping-pong grids (C, K, N...)
-        op->T.alloc(es * (size_t)op->C * op->K * op->V);
-        op->T2.alloc(es * (size_t)op->C * op->K * op->V);
-    } else if (!op->fused) {  // two ping-pong grids (Cb, K, 2N...)
-        op->T.alloc(lines_scratch_bytes(op, es));
-        op->T2.alloc(lines_scratch_bytes(op, es));
+    if (op->cart || !op->fused) {
+        op->T.alloc(es * general_scratch(op, 0));
+        op->T2.alloc(es * general_scratch(op, 1));
     } else if (op->d == 2) {
         op->T.alloc(es * (size_t)op->C * op->K * (2 * nx) * ny);
     } else {
@@ -223,7 +237,8 @@ void op_set_cmaps(msr_normalop* op, int ncoils, const void* const* cmaps, hipStr
 
 GridDims op_grid(const msr_normalop* op) {
     const int pad = op->cart ? 1 : 2;
-    GridDims g{{pad * op->N[0], pad * op->N[1], op->d == 3 ? pad * op->N[2] : 1}, op->cart};
+    GridDims g{{pad * op->N[0], pad * op->N[1], op->d == 3 ? pad * op->N[2] : 1},
+               op->cart && !op->planes};
     return g;
 }
 
@@ -283,9 +298,12 @@ msr_normalop* op_new(msr_ctx* ctx, int d, const int64_t* N, int K, int lam_real,
     op->P = cart ? K * K : K * (K + 1) / 2;
     op->lam_real = lam_real;
     op->cart = cart ? 1 : 0;
-    // MSR_APPLY_LINES=1 sends every non-Cartesian operator to the line-kernel
-    // apply (a cross-check of the two paths on shapes both cover)
-    op->fused = !cart && fused_shape(d, N, K) && env_int("MSR_APPLY_LINES", 0) == 0;
+    // cross-checks of the paths on shapes several of them cover:
+    // MSR_APPLY_PLANES=1 sends every non-Cartesian operator past the fused
+    // passes to the fused line passes, MSR_APPLY_LINES=1 to the separate ones
+    const bool lines = env_int("MSR_APPLY_LINES", 0) != 0;
+    op->fused = !cart && fused_shape(d, N, K) && !lines && env_int("MSR_APPLY_PLANES", 0) == 0;
+    op->planes = !op->fused && planes_supported(d, N, cart ? 1 : 2, K) && (cart || !lines);
     return op.release();
 }
 
@@ -330,7 +348,9 @@ void op_passes(msr_normalop* op, const void* b, int am, hipStream_t st, const in
     const bool f64 = am != AM_F32;
     MSR_REQUIRE(op->scratch_es >= (f64 ? sizeof(double2) : sizeof(float2)), MSR_ERR_ERROR,
                 "apply scratch not allocated for this precision");
-    if (op->cart) {
+    if (op->planes) {
+        launch_planes_passes(op, b, f64, st, skip, 0, op->C, op->G);
+    } else if (op->cart) {
         launch_cart_passes(op, b, f64, st, skip);
     } else if (!op->fused) {
         launch_lines_passes(op, b, f64, st, skip);
@@ -366,7 +386,9 @@ void op_apply_percoil(msr_normalop* op, float2* x, const float2* b, float2 alpha
                 "the per-coil apply order exists for the non-Cartesian operator only");
     launch_scale<float2>(x, op->V * op->K, beta, beta_zero, st);
     for (int c = 0; c < op->C; ++c) {
-        if (!op->fused) {
+        if (op->planes) {
+            launch_planes_passes(op, b, false, st, nullptr, c, c + 1, 1);
+        } else if (!op->fused) {
             launch_lines_passes(op, b, false, st, nullptr, c, c + 1);
         } else if (op->d == 2) {
             Apply2DArgs a = args2d(op, AM_F32);
@@ -415,8 +437,7 @@ size_t op_footprint(const msr_normalop* op, int prec) {
     const size_t vs = v64 ? sizeof(double2) : sizeof(float2);  // CG vectors
     const int64_t nx = op->N[0], ny = op->N[1], nz = op->N[2];
     size_t scratch = es * (size_t)op->G * op->K * op->V;
-    if (op->cart) scratch += 2 * es * (size_t)op->C * op->K * op->V;
-    else if (!op->fused) scratch += 2 * lines_scratch_bytes(op, es);
+    if (op->cart || !op->fused) scratch += es * (general_scratch(op, 0) + general_scratch(op, 1));
     else if (op->d == 2) scratch += es * (size_t)op->C * op->K * (2 * nx) * ny;
     else scratch += es * (size_t)op->C * op->K * nz * ny * 2 * nx * 3;  // T1 + T2
     size_t cg = vs * n * 2 + es * n;                                   // r, u, c

@@ -20,7 +20,7 @@ void launch_cart_passes(msr_normalop* op, const void* b, bool f64, hipStream_t s
 void launch_lines_passes(msr_normalop* op, const void* b, bool f64, hipStream_t st,
                          const int* skip, int c_begin = 0, int c_end = -1);
 int lines_chunk_coils(const msr_normalop* op);
-size_t lines_scratch_bytes(const msr_normalop* op, size_t es);
+size_t general_scratch(const msr_normalop* op, int which);  // elements of T (0) / T2 (1)
 // the largest coefficient count (the fused passes take up to 8)
 constexpr int MAX_COEFFS = 64;
 void op_set_cmaps(msr_normalop* op, int ncoils, const void* const* cmaps, hipStream_t st);

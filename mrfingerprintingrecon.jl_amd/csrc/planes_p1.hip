@@ -1,0 +1,10 @@
+// Fused line passes for the lengths of part 1 (MSR_FFT_LINE_LENGTHS_P1).
+#include "planes_impl.hpp"
+
+namespace msr {
+
+bool plane_part1(int which, const PlanePass& p, const void* tw, hipStream_t st) {
+    MSR_PLANE_PART_BODY(MSR_FFT_LINE_LENGTHS_P1)
+}
+
+}  // namespace msr

@@ -1,0 +1,10 @@
+// Fused line passes for the lengths of part 3 (MSR_FFT_LINE_LENGTHS_P3).
+#include "planes_impl.hpp"
+
+namespace msr {
+
+bool plane_part3(int which, const PlanePass& p, const void* tw, hipStream_t st) {
+    MSR_PLANE_PART_BODY(MSR_FFT_LINE_LENGTHS_P3)
+}
+
+}  // namespace msr
