@@ -2,15 +2,22 @@
 // reference tests (test/reconstruct_radial.jl:62-74: for every coil and frame,
 // NonuniformFFTs exec_type2! of S_c * sum_k U[t, k] x_k):
 //   y_{j,c} = sum_k U[t_j, k] sum_n S_c[n] x_k[n] exp(-2 pi i k_j . (n - N/2))
-// On the device: z_{c,k} = S_c x_k; centred placement on the sigma = 2 grid with
-// deapodisation 1/phihat fused into the first line pass; forward FFTs; then ES
-// interpolation (W = 8) at the samples, where each lane of a wavefront owns one
-// kernel cell, folds the K channels with U[t_j, k] in registers, and the
-// wavefront reduces the 64 (8x8, z looped in 3D) cell contributions.
+// On the device: S_c x_k, centred placement on the sigma = 2 grid with
+// deapodisation 1/phihat, forward FFTs, then ES interpolation (W = 8) at the
+// samples.  Two forms of the interpolation:
+//  - 2D, on the matrix cores (interp_mfma_kernel): samples sorted by region of
+//    4 x 5 cells, 16 samples of one region at a time;
+//  - one wavefront per sample (interp_kernel: 3D, and the shapes the rule in
+//    fwd_batches_pay leaves): each lane owns one kernel cell, folds the K
+//    channels with U[t_j, k] in registers, and the wavefront reduces the 64
+//    (8x8, z looped in 3D) cell contributions.
 #include <algorithm>
+
+#include <hipcub/hipcub.hpp>
 
 #include "fft.hpp"
 #include "fftlines.hpp"
+#include "planes.hpp"
 #include "spread.hpp"
 
 namespace msr {
@@ -141,6 +148,218 @@ interp_kernel(const float* __restrict__ kc, const int* __restrict__ frame,
     }
 }
 
+// --------------------------------------------- 2D on the matrix cores
+// A region is 4 x 5 cells; the kernels of the samples whose floor cell lies in
+// it reach 11 x 12 cells (rows qx, columns qy).  One wavefront takes 16 samples
+// of a region (the MFMA's columns) and, group by group of 8 coils, the product
+//   Z (16 floats: 8 coils re/im x 16 samples) = G (16 x 132 cells) W (132 x 16)
+// as 33 v_mfma_f32_16x16x4f32, four neighbouring cells along qy per step: lane
+// (r = lane mod 16, s = lane div 16) supplies float r of cell s (the grid is
+// stored [k][coil group][qx][qy][8 coils], so a step's 64 lanes read 256
+// consecutive bytes) and the weight w_x w_y of cell s for sample r.  Each
+// accumulator holds two coils of one sample and is folded with U[t_j, k] before
+// the next coefficient.  A step's grid values are loaded one (coil group,
+// coefficient) ahead.
+//
+// Bound: matrix-core issue (33 x 32 cycles per 16 samples, coefficient and 8
+// coils; the 64 cells of a kernel are 48 % of the region's 132, and a region
+// away from the centre fills about 12 of the 16 columns).  At 256 x 256, 20
+// coils, K = 5, 512 000 samples on MI355X: interpolation
+// 3.43 -> 0.55 ms, a call with its FFTs 4.11 -> 0.68 ms
+constexpr int FW_TX = 4, FW_TY = 5;                      // region (floor cells)
+constexpr int FW_RX = FW_TX + 7, FW_RY = (FW_TY + 7) / 4;  // rows, column quads it reaches
+constexpr int FW_STEPS = FW_RX * FW_RY;
+static_assert(FW_RY * 4 == FW_TY + 7, "the columns of a region come in quads");
+constexpr int FW_PTS = 16;                               // samples per batch
+
+__global__ void fwd_region_kernel(const float* __restrict__ kc, int64_t M, FwdGeom g, int nry,
+                                  int* __restrict__ key, int* __restrict__ idx) {
+    for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < M;
+         j += (int64_t)gridDim.x * blockDim.x) {
+        int64_t cx, cy;
+        float f;
+        cell_frac(kc[2 * j], g.n[0], cx, f);
+        cell_frac(kc[2 * j + 1], g.n[1], cy, f);
+        key[j] = (int)(cx / FW_TX) * nry + (int)(cy / FW_TY);
+        idx[j] = (int)j;
+    }
+}
+
+// first position of a sorted key >= v
+__device__ __forceinline__ int lower_bound(const int* __restrict__ sorted, int n, int v) {
+    int lo = 0, hi = n;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sorted[mid] < v) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// first[r] = first sample of region r (r <= nr), nb[r] = its batches
+__global__ void fwd_count_kernel(const int* __restrict__ sorted, int M, int nr, int* __restrict__ first,
+                                 int* __restrict__ nb) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r > nr) return;
+    const int a = lower_bound(sorted, M, r);
+    first[r] = a;
+    nb[r] = r < nr ? (lower_bound(sorted, M, r + 1) - a + FW_PTS - 1) / FW_PTS : 0;
+}
+
+// batch b -> {region, first sample, samples}
+__global__ void fwd_batch_kernel(const int* __restrict__ first, const int* __restrict__ pos, int nr, int nbatch,
+                                 int4* __restrict__ batches) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= nbatch) return;
+    const int r = lower_bound(pos, nr + 1, b + 1) - 1;  // pos[r] <= b < pos[r + 1]
+    const int s = first[r] + (b - pos[r]) * FW_PTS;
+    const int left = first[r + 1] - s;
+    batches[b] = make_int4(r, s, left < FW_PTS ? left : FW_PTS, 0);
+}
+
+// Samples sorted by region (stable) and cut into batches, once per trajectory
+// and grid.
+static const FwdPlan& fwd_plan(const msr_traj* traj, const FwdGeom& g, hipStream_t st) {
+    std::array<int64_t, 2> key{g.n[0], g.n[1]};
+    auto it = traj->fwd_plans.find(key);
+    if (it != traj->fwd_plans.end()) return *it->second;
+    MSR_REQUIRE(traj->M < (int64_t)INT32_MAX, MSR_ERR_UNSUPPORTED, "more than 2^31 samples");
+    auto p = std::make_unique<FwdPlan>();
+    const int M = (int)traj->M;
+    p->nry = (int)ceil_div(g.n[1], FW_TY);
+    const int nr = (int)ceil_div(g.n[0], FW_TX) * p->nry;
+    DevBuf keys, sorted, idx, temp, first, nb, pos;
+    keys.alloc(sizeof(int) * M);
+    sorted.alloc(sizeof(int) * M);
+    idx.alloc(sizeof(int) * M);
+    p->perm.alloc(sizeof(int) * M);
+    first.alloc(sizeof(int) * (nr + 1));
+    nb.alloc(sizeof(int) * (nr + 1));
+    pos.alloc(sizeof(int) * (nr + 1));
+    const int grid = (int)std::min<int64_t>((traj->M + 255) / 256, 8192);
+    hipLaunchKernelGGL(fwd_region_kernel, dim3(grid), dim3(256), 0, st, traj->kc.as<float>(), traj->M, g,
+                       p->nry, keys.as<int>(), idx.as<int>());
+    MSR_CHECK_LAUNCH();
+    int bits = 1;
+    while ((int64_t(1) << bits) < nr) ++bits;
+    size_t tb = 0, ts = 0;
+    MSR_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, keys.as<int>(), sorted.as<int>(), idx.as<int>(),
+                                               p->perm.as<int>(), M, 0, bits, st));
+    MSR_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, ts, nb.as<int>(), pos.as<int>(), nr + 1, st));
+    temp.alloc(std::max<size_t>(std::max(tb, ts), 16));
+    MSR_HIP(hipcub::DeviceRadixSort::SortPairs(temp.p, tb, keys.as<int>(), sorted.as<int>(), idx.as<int>(),
+                                               p->perm.as<int>(), M, 0, bits, st));
+    hipLaunchKernelGGL(fwd_count_kernel, dim3((nr + 256) / 256), dim3(256), 0, st, sorted.as<int>(), M, nr,
+                       first.as<int>(), nb.as<int>());
+    MSR_CHECK_LAUNCH();
+    MSR_HIP(hipcub::DeviceScan::ExclusiveSum(temp.p, ts, nb.as<int>(), pos.as<int>(), nr + 1, st));
+    MSR_HIP(hipMemcpyAsync(&p->nbatch, pos.as<int>() + nr, sizeof(int), hipMemcpyDeviceToHost, st));
+    MSR_HIP(hipStreamSynchronize(st));
+    p->batches.alloc(sizeof(int4) * std::max(p->nbatch, 1));
+    hipLaunchKernelGGL(fwd_batch_kernel, dim3((p->nbatch + 255) / 256), dim3(256), 0, st, first.as<int>(),
+                       pos.as<int>(), nr, p->nbatch, p->batches.as<int4>());
+    MSR_CHECK_LAUNCH();
+    MSR_HIP(hipStreamSynchronize(st));  // temporaries are freed on return
+    auto& ref = *p;
+    traj->fwd_plans[key] = std::move(p);
+    return ref;
+}
+
+using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
+
+__global__ void __launch_bounds__(256)
+interp_mfma_kernel(const float* __restrict__ kc, const int* __restrict__ frame, const int64_t* __restrict__ sel,
+                   const int* __restrict__ perm, const int4* __restrict__ batches, int nbatch, int nry,
+                   int64_t nsel, const float* __restrict__ G, FwdGeom g, int K, int C,
+                   const void* __restrict__ U, int u_real, int64_t nt, float2* __restrict__ out) {
+    // consecutive batches (neighbouring regions) on one XCD
+    const int nblk = gridDim.x;
+    const int lb = nblk % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (nblk / 8) + (int)blockIdx.x / 8;
+    const int wv = __builtin_amdgcn_readfirstlane(lb * 4 + (threadIdx.x >> 6));
+    if (wv >= nbatch) return;
+    const int lane = threadIdx.x & 63, r = lane & 15, s = lane >> 4;
+    const int4 bt = batches[wv];
+    const int X0 = bt.x / nry * FW_TX - 3, Y0 = bt.x % nry * FW_TY - 3;  // first cell reached
+    const bool on = r < bt.z;
+    const int64_t j = perm[bt.y + (on ? r : 0)];
+    int64_t cx, cy;
+    float fx, fy;
+    cell_frac(kc[2 * j], g.n[0], cx, fx);
+    cell_frac(kc[2 * j + 1], g.n[1], cy, fy);
+    const int t = frame[j];
+    const int64_t idx = sel ? sel[j] : j;
+    const int n0 = (int)g.n[0], n1 = (int)g.n[1];
+    float wx[FW_RX], wy[FW_RY];
+    int oy[FW_RY];
+#pragma unroll
+    for (int i = 0; i < FW_RX; ++i) wx[i] = on ? es_phi_fw((float)(X0 + i - (int)cx) - fx) : 0.f;
+#pragma unroll
+    for (int q = 0; q < FW_RY; ++q) {
+        const int y = Y0 + 4 * q + s;
+        wy[q] = es_phi_fw((float)(y - (int)cy) - fy);
+        oy[q] = ((y % n1 + n1) % n1) * (2 * PLANE_COIL_GROUP) + r;  // float of the cell
+    }
+    const int CB = (C + PLANE_COIL_GROUP - 1) / PLANE_COIL_GROUP, ng = CB * K;
+    const int64_t plane = (int64_t)n0 * n1 * (2 * PLANE_COIL_GROUP);
+    const int row = n1 * 2 * PLANE_COIL_GROUP;
+    float a[FW_STEPS];
+    // group q = cb K + k
+    auto base = [&](int q) { return G + ((int64_t)(q % K) * CB + q / K) * plane; };
+    auto load = [&](const float* b, int st) {
+        const int x = X0 + st / FW_RY;
+        return b[(int64_t)((x % n0 + n0) % n0) * row + oy[st % FW_RY]];
+    };
+    const float* b0 = base(0);
+#pragma unroll
+    for (int st = 0; st < FW_STEPS; ++st) a[st] = load(b0, st);
+    float2 y[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+    int k = 0, cb = 0;
+    for (int q = 0; q < ng; ++q) {
+        const float* nb = base(q + 1 < ng ? q + 1 : q);
+        float2 u;
+        if (u_real) u = make_float2(reinterpret_cast<const float*>(U)[t + (int64_t)k * nt], 0.f);
+        else u = reinterpret_cast<const float2*>(U)[t + (int64_t)k * nt];
+        f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st < FW_STEPS; ++st) {
+            z = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st], wx[st / FW_RY] * wy[st % FW_RY], z, 0, 0, 0);
+            a[st] = load(nb, st);
+        }
+        cfma(y[0], u, make_float2(z[0], z[1]));
+        cfma(y[1], u, make_float2(z[2], z[3]));
+        if (++k == K) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int c = cb * PLANE_COIL_GROUP + 2 * s + h;
+                if (on && c < C) out[idx + (int64_t)c * nsel] = y[h];
+                y[h] = make_float2(0.f, 0.f);
+            }
+            k = 0;
+            ++cb;
+        }
+    }
+}
+
+// Whether the batches pay: a batch costs the same however many samples it
+// holds, 0.43 ns per coefficient and 8 coils at full rate against 0.27 ns per
+// sample, coefficient and 4 coils of the one-wavefront-per-sample kernel
+// (measured 3.43 ms at 512 000 samples, 20 coils, K = 5).  From 4 coils on: the
+// grid is stored for whole groups of 8.
+static bool fwd_batches_pay(int64_t nbatch, int64_t M, int C) {
+    return C >= 4 && 8 * nbatch * ceil_div(C, 8) <= 5 * M * ceil_div(C, 4);
+}
+
+// Device copy of the coil maps, packed (C, V): one launch per 32 coils.
+constexpr int FW_MAPS = 32;
+struct FwdMaps {
+    const float2* p[FW_MAPS];
+};
+__global__ void pack_maps_kernel(FwdMaps m, int64_t V, float2* __restrict__ out) {
+    const float2* src = m.p[blockIdx.y];
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < V; v += (int64_t)gridDim.x * blockDim.x)
+        out[(int64_t)blockIdx.y * V + v] = src[v];
+}
+
 void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, const void* x,
                    int K, const void* U, int u_real, int ncoils, const void* const* cmaps, void* out,
                    hipStream_t st) {
@@ -161,24 +380,73 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
         Gos *= nos[a];
     }
     const int nch = C * K;
-    // workspace: Z (nch*V) and two grid buffers
-    DevBuf work;
-    const size_t zb = sizeof(float2) * (size_t)nch * V, gb = sizeof(float2) * (size_t)nch * Gos;
-    work.alloc(zb + 2 * gb);
-    float2* Z = work.as<float2>();
-    float2* A = reinterpret_cast<float2*>(reinterpret_cast<char*>(work.p) + zb);
-    float2* B = reinterpret_cast<float2*>(reinterpret_cast<char*>(work.p) + zb + gb);
-    // pack the coil maps (C device pointers) into one buffer when given
-    DevBuf maps;
-    const float2* mp = nullptr;
-    if (ncoils >= 1 && cmaps) {
-        maps.alloc(sizeof(float2) * (size_t)C * V);
-        for (int c = 0; c < C; ++c) {
-            MSR_REQUIRE(cmaps[c] != nullptr, MSR_ERR_ARGUMENT, "cmaps[%d] is NULL", c);
-            MSR_HIP(hipMemcpyAsync(maps.as<float2>() + (size_t)c * V, cmaps[c], sizeof(float2) * V,
-                                   hipMemcpyDeviceToDevice, st));
+    // the plan and the workspace belong to the handle: hold it until the call's
+    // kernels have run (allocated and freed on every call, the workspace took up to
+    // 12 ms of a call with 3.9 ms of kernels)
+    std::lock_guard<std::recursive_mutex> lock(traj->mu);
+    const FwdGeom g{{nos[0], nos[1], nos[2]}};
+    const FwdPlan* plan = nullptr;
+    if (d == 2 && U && nos[0] <= 1024 && nos[1] <= 1024 && traj->M > 0) {
+        plan = &fwd_plan(traj, g, st);
+        if (!fwd_batches_pay(plan->nbatch, traj->M, C)) plan = nullptr;
+    }
+    const int CB = (int)ceil_div(C, PLANE_COIL_GROUP);
+    const bool maps = ncoils >= 1 && cmaps;
+    const size_t mb = maps ? (sizeof(float2) * (size_t)C * V + 255) / 256 * 256 : 0;
+    // workspace: coil maps, then S_c x_k and two grid buffers, or (matrix
+    // cores) the row transforms and the grid in groups of 8 coils
+    const size_t zb = plan ? 0 : sizeof(float2) * (size_t)nch * V;
+    const size_t ab = plan ? (sizeof(float2) * (size_t)nch * nos[0] * NN[1] + 255) / 256 * 256
+                           : sizeof(float2) * (size_t)nch * Gos;
+    const size_t bb = plan ? sizeof(float2) * (size_t)K * CB * PLANE_COIL_GROUP * Gos : ab;
+    DevBuf& work = traj->fwd_work;
+    if (work.bytes < mb + zb + ab + bb) work.alloc(mb + zb + ab + bb);
+    float2* mp = maps ? work.as<float2>() : nullptr;
+    float2* Z = reinterpret_cast<float2*>(work.as<char>() + mb);
+    float2* A = reinterpret_cast<float2*>(work.as<char>() + mb + zb);
+    float2* B = reinterpret_cast<float2*>(work.as<char>() + mb + zb + ab);
+    if (maps)
+        for (int c0 = 0; c0 < C; c0 += FW_MAPS) {
+            FwdMaps m{};
+            const int nc = std::min(FW_MAPS, C - c0);
+            for (int c = 0; c < nc; ++c) {
+                MSR_REQUIRE(cmaps[c0 + c] != nullptr, MSR_ERR_ARGUMENT, "cmaps[%d] is NULL", c0 + c);
+                m.p[c] = (const float2*)cmaps[c0 + c];
+            }
+            hipLaunchKernelGGL(pack_maps_kernel, dim3((unsigned)std::min<int64_t>((V + 255) / 256, 1024), nc),
+                               dim3(256), 0, st, m, V, mp + (int64_t)c0 * V);
+            MSR_CHECK_LAUNCH();
         }
-        mp = maps.as<float2>();
+    const int64_t nsel = traj->nsamp * traj->nt;
+    if (traj->sel.p) fill_floats(out, 2 * nsel * C, 0.f, st);  // masked-out samples are 0
+    if (plan) {
+        PlanePass px;
+        px.nf = (int)nos[0];
+        px.len = (int)NN[0];
+        px.K = K;
+        px.nc = C;
+        px.T = A;
+        px.plane = nos[0] * NN[1];
+        px.nrows = NN[1];
+        px.b = x;
+        px.cmaps = mp;
+        px.win = deapod_table(ctx, (int)nos[0], (int)NN[0], SEL_CENTER);
+        run_plane(PLANE_PLACE, px, ctx, st);
+        PlanePass py = px;
+        py.nf = (int)nos[1];
+        py.len = (int)NN[1];
+        py.ncols = nos[0];
+        py.out = B;
+        py.win = deapod_table(ctx, (int)nos[1], (int)NN[1], SEL_CENTER);
+        run_plane(PLANE_COILS, py, ctx, st);
+        hipLaunchKernelGGL(interp_mfma_kernel, dim3((plan->nbatch + 3) / 4), dim3(256), 0, st,
+                           traj->kc.as<float>(), traj->frame.as<int>(),
+                           traj->sel.p ? traj->sel.as<int64_t>() : nullptr, plan->perm.as<int>(),
+                           plan->batches.as<int4>(), plan->nbatch, plan->nry, nsel,
+                           reinterpret_cast<const float*>(B), g, K, C, U, u_real, traj->nt, (float2*)out);
+        MSR_CHECK_LAUNCH();
+        MSR_HIP(hipStreamSynchronize(st));  // the workspace is free again
+        return;
     }
     int grid = (int)std::min<int64_t>(((int64_t)nch * V + 255) / 256, 16384);
     hipLaunchKernelGGL(expand_kernel, dim3(grid), dim3(256), 0, st, (const float2*)x, mp, C, K, V, Z);
@@ -238,9 +506,6 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
         run_cols(pz, ctx, st);
         Gfin = A;
     }
-    const int64_t nsel = traj->nsamp * traj->nt;
-    if (traj->sel.p) fill_floats(out, 2 * nsel * C, 0.f, st);  // masked-out samples are 0
-    FwdGeom g{{nos[0], nos[1], nos[2]}};
     const int64_t waves = traj->M;
     const int blocks = (int)std::min<int64_t>((waves * 64 + 255) / 256, 65536);
     if (d == 2)
@@ -252,7 +517,7 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
                            traj->frame.as<int>(), traj->sel.p ? traj->sel.as<int64_t>() : nullptr,
                            traj->M, nsel, Gfin, g, K, C, U, u_real, traj->nt, (float2*)out);
     MSR_CHECK_LAUNCH();
-    MSR_HIP(hipStreamSynchronize(st));  // workspace is freed on return
+    MSR_HIP(hipStreamSynchronize(st));  // the workspace is free again
 }
 
 }  // namespace msr

@@ -104,6 +104,14 @@ struct CartPlan {
     DevBuf offs;                // (G + 1) int32
 };
 
+// Region sort of a trajectory's samples for the 2D forward model (forward.hip):
+// batches of up to 16 samples of one region.
+struct FwdPlan {
+    int nry = 0, nbatch = 0;    // regions along y, batches
+    DevBuf perm;                // (M) int32: samples sorted by region
+    DevBuf batches;             // (nbatch) int4 {region, first sorted sample, samples, 0}
+};
+
 // CG scalar state kept on the device (FP64).
 struct CgScalars {
     double res, prev, tol;
@@ -125,6 +133,8 @@ struct msr_traj {
     std::vector<int64_t> nsamp_t;     // host copy of the per-frame counts
     mutable std::map<std::array<int64_t, 3>, std::unique_ptr<msr::SpreadPlan>> plans;
     mutable msr::DevBuf bp_work;      // backprojection workspace (grow-only)
+    mutable msr::DevBuf fwd_work;     // forward-model workspace (grow-only)
+    mutable std::map<std::array<int64_t, 2>, std::unique_ptr<msr::FwdPlan>> fwd_plans;
     bool integer = false;             // created from integer (Cartesian) k-space indices
     mutable std::map<std::array<int64_t, 3>, std::unique_ptr<msr::CartPlan>> cart_plans;
     // The plan maps and the workspace are shared by every call on the handle:

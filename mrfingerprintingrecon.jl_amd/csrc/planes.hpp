@@ -22,7 +22,7 @@
 
 namespace msr {
 
-enum { PLANE_EXPAND = 0, PLANE_MULTIPLY = 1, PLANE_COMBINE = 2 };
+enum { PLANE_EXPAND = 0, PLANE_MULTIPLY = 1, PLANE_COMBINE = 2, PLANE_PLACE = 3, PLANE_COILS = 4 };
 
 struct PlanePass {
     int f64 = 0;
@@ -43,9 +43,17 @@ struct PlanePass {
     int64_t ncols = 0, cs = 0, es = 0;
     const void* lam = nullptr;     // lam[(col * P + p) * nf + i]
     int lam_real = 0, lam_full = 0;// Float32; P = K * K entries j + K k (else packed Hermitian)
+    // forward model (ComplexF32): rows placed around frequency zero and scaled
+    // (place), then lines along y of PLANE_COIL_GROUP coils at a time (coils):
+    // T[(k nc + c) plane + q nrows + row] -> out[((k CB + c / 8) ncols + col) nf + q][c % 8]
+    const float* win = nullptr;    // deapodisation of the stored elements
+    float2* out = nullptr;
     const int* skip = nullptr;
 };
 
+constexpr int PLANE_COIL_GROUP = 8;  // coils side by side: 64 bytes of a cell
+
+// Place and coils passes cover nf <= 1024 on both axes.
 // Launches one pass (twiddles from the context's tables).
 void run_plane(int which, const PlanePass& p, msr_ctx* ctx, hipStream_t st);
 

@@ -325,6 +325,68 @@ plane_multiply_kernel(PlanePass p, const CT* __restrict__ tw, int wcs) {
         });
 }
 
+// ---------------------------------------------------------- forward model
+// Stored element of FFT bin q when the len elements are centred on frequency
+// zero (element len/2 in bin 0), or >= len in the padding.
+template <int NF>
+__device__ __forceinline__ int plane_centred(int q, int len) {
+    const int i = q + len / 2;
+    return i >= NF ? i - NF : i;
+}
+
+// Block = (row tile, k, c): rows of S_c x_k, placed, deapodised and transformed
+// along x, written transposed.
+template <int NF>
+__global__ void __launch_bounds__((plane_row_block<NF, float2>()))
+plane_place_kernel(PlanePass p, const float2* __restrict__ tw) {
+    constexpr int F = plane_rows<NF, float2>(), SH = plane_shift(F), BLK = plane_row_block<NF, float2>();
+    constexpr int LP = plane_pitch<NF, float2>();
+    __shared__ float2 s[F * LP];
+    const int64_t tiles = (p.nrows + F - 1) / F;
+    const int64_t lb = plane_xcd(blockIdx.x, tiles * p.K * p.nc);
+    const int c = (int)(lb % p.nc), k = (int)((lb / p.nc) % p.K);
+    const int64_t r0 = lb / ((int64_t)p.nc * p.K) * F;
+    const int nr = (int)(p.nrows - r0 < F ? p.nrows - r0 : F), len = p.len;
+    const float2* b = static_cast<const float2*>(p.b) + ((int64_t)k * p.nrows + r0) * len;
+    const float2* cm = p.cmaps ? p.cmaps + ((int64_t)c * p.nrows + r0) * len : nullptr;
+    float2* T = static_cast<float2*>(p.T) + ((int64_t)k * p.nc + c) * p.plane + r0;
+    plane_fft<NF, -1, 0, 1, true, false, float2>(s, F, tw, false, false, SH,
+        [&](int l, int q) {
+            const int i = plane_centred<NF>(q, len);
+            if (i >= len || l >= nr) return make_float2(0.f, 0.f);
+            const float2 v = b[l * len + i];
+            return cscale(cm ? cmul(cm[l * len + i], v) : v, p.win[i]);
+        },
+        [](int, int, int, int, float2) {});
+    for (int e = threadIdx.x; e < F * NF; e += BLK) {
+        const int q = e >> SH, l = e & (F - 1);
+        if (l < nr) T[l + (int64_t)q * p.nrows] = s[l * LP + plane_at<NF, float2>(q)];
+    }
+}
+
+// Block = (k, coil group, column): the group's lines along y, placed and
+// transformed, written with the coils side by side.
+template <int NF>
+__global__ void __launch_bounds__(1024) plane_coils_kernel(PlanePass p, const float2* __restrict__ tw) {
+    constexpr int F = PLANE_COIL_GROUP, LP = plane_pitch<NF, float2>();
+    __shared__ float2 s[F * LP];
+    const int CB = (p.nc + F - 1) / F, len = p.len;
+    const int64_t lb = plane_xcd(blockIdx.x, p.ncols * CB * p.K);
+    const int64_t col = lb % p.ncols, g = lb / p.ncols;  // g = k CB + coil group
+    const int k = (int)(g / CB), c0 = (int)(g % CB) * F;
+    const float2* T = static_cast<const float2*>(p.T) + ((int64_t)k * p.nc + c0) * p.plane + col * len;
+    plane_fft<NF, -1, 0, 1, true, false, float2>(s, F, tw, false, false, 3,
+        [&](int l, int q) {
+            const int i = plane_centred<NF>(q, len);
+            if (i >= len || c0 + l >= p.nc) return make_float2(0.f, 0.f);
+            return cscale(T[l * p.plane + i], p.win[i]);
+        },
+        [](int, int, int, int, float2) {});
+    float2* out = p.out + (g * p.ncols + col) * NF * F;
+    for (int e = threadIdx.x; e < F * NF; e += blockDim.x)
+        out[e] = s[(e & (F - 1)) * LP + plane_at<NF, float2>(e / F)];
+}
+
 // ---------------------------------------------------------------- launch
 inline unsigned plane_grid(int64_t n) {
     MSR_REQUIRE(n >= 1 && n < (int64_t)1 << 31, MSR_ERR_ARGUMENT, "launch of %lld blocks", (long long)n);
@@ -333,6 +395,24 @@ inline unsigned plane_grid(int64_t n) {
 
 template <int NF, class CT>
 void launch_plane_n(int which, const PlanePass& p, const CT* tw, hipStream_t st) {
+    if (which == PLANE_PLACE || which == PLANE_COILS) {
+        if constexpr (sizeof(CT) == 8 && NF <= PLANE_MAX_ROW) {
+            if (which == PLANE_PLACE) {
+                const int64_t tiles = ceil_div(p.nrows, plane_rows<NF, CT>());
+                constexpr int BLK = plane_row_block<NF, CT>();
+                hipLaunchKernelGGL((plane_place_kernel<NF>), dim3(plane_grid(tiles * p.K * p.nc)), dim3(BLK),
+                                   0, st, p, tw);
+            } else {
+                constexpr int BLK = (PLANE_COIL_GROUP * NF + PLANE_VALUES - 1) / PLANE_VALUES;
+                hipLaunchKernelGGL((plane_coils_kernel<NF>),
+                                   dim3(plane_grid(p.ncols * ceil_div(p.nc, PLANE_COIL_GROUP) * p.K)),
+                                   dim3((BLK + 63) / 64 * 64), 0, st, p, tw);
+            }
+        } else {
+            fail(MSR_ERR_ERROR, "forward-model pass of length %d", NF);
+        }
+        return;
+    }
     if (which == PLANE_MULTIPLY) {
         // columns per block: strided ones 64 bytes of neighbours, contiguous
         // ones up to 256 threads; fewer while the block would leave room for
