@@ -1,0 +1,94 @@
+"""Kernel construction against the FP64 oracle at the edges of its spreading
+(output tiles of 4 cells per dimension, runs of bins that wrap, 1 to 10 row
+tiles of pair products) and of its mask: grids of one, two and three bins,
+ragged sizes, one sample, samples on the grid's edge, real and complex bases.
+The mask is bit-exact, the kernel within 3e-7 (W = 8 spreading, rounded to
+ComplexF32), and a construction repeats bit for bit, alone or beside others on
+threads and streams of their own (whose temporaries share recycled memory)."""
+import threading
+
+import numpy as np
+import pytest
+
+from conftest import load_package, rel_err
+from oracle import toeplitz
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return torch
+
+
+@pytest.fixture(scope="module")
+def msr():
+    return load_package()
+
+
+def protocol(N, K, nt, ns, real, seed=0):
+    rng = np.random.default_rng(seed)
+    trj = rng.uniform(-0.5, 0.5, size=(nt, ns, len(N))).astype(np.float32)
+    trj[0, 0] = -0.5
+    if ns > 2:
+        trj[0, 1] = 0.5
+        trj[:, 2:ns // 2] *= np.float32(0.02)  # a dense centre: many samples per tile
+    U = rng.normal(size=(K, nt)) + (0 if real else 1j * rng.normal(size=(K, nt)))
+    return trj, U.astype(np.float32 if real else np.complex64)
+
+
+CASES = [
+    ((1, 2), 2, 3, 40, False),       # 4N = 4 x 8: below three bins
+    ((3, 3), 1, 2, 1, False),        # 12 x 12: three bins, two samples
+    ((3, 5), 3, 5, 300, True),
+    ((4, 9), 4, 6, 200, False),      # P = 10: two row tiles
+    ((16, 15), 12, 4, 100, False),   # P = 78: three groups of four tiles
+    ((15, 16), 9, 4, 100, True),     # P = 45 real: three tiles in a group of four
+    ((64, 48), 5, 20, 400, False),
+    ((3, 4, 5), 3, 4, 300, False),
+    ((5, 3, 3), 4, 3, 100, True),
+    ((12, 10, 9), 2, 6, 500, False),
+]
+
+
+@pytest.mark.parametrize("N,K,nt,ns,real", CASES)
+def test_kernel_matches_oracle(torch, msr, N, K, nt, ns, real):
+    trj, U = protocol(N, K, nt, ns, real)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    A = msr.NFFTNormalOp(N, dev(trj), dev(U))
+    ref, km = toeplitz.toeplitz_kernel(N, trj, U)
+    assert np.array_equal(A.prod.A.kmask_indcs.cpu().numpy() - 1, km)
+    lam = A.prod.A.Λ
+    e = rel_err(lam.cpu().numpy(), ref)
+    print(f"kernel {N} K={K} real={real}: {e:.2e}", flush=True)
+    assert e < 3e-7
+    again = msr.NFFTNormalOp(N, dev(trj), dev(U)).prod.A.Λ
+    assert torch.equal(lam, again)
+
+
+def test_constructions_on_threads_and_streams(torch, msr):
+    jobs = [((24, 20), 3), ((12, 10, 9), 2), ((32, 27), 4), ((16, 16), 5)]
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    inputs = [[dev(a) for a in protocol(N, K, 8, 200, False, seed=i)] for i, (N, K) in enumerate(jobs)]
+    want = [msr.NFFTNormalOp(N, *inp).prod.A.Λ for (N, K), inp in zip(jobs, inputs)]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            for _ in range(5):
+                got = msr.NFFTNormalOp(jobs[i][0], *inputs[i]).prod.A.Λ
+                st.synchronize()
+                if not torch.equal(got, want[i]):
+                    wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
