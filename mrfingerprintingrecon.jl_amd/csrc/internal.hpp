@@ -35,25 +35,34 @@ struct msr_ctx {
 
 namespace msr {
 
+// Device memory behind DevBuf (devbuf.hip): blocks of freed buffers are kept,
+// up to a bounded number of idle bytes per device, and handed out again.
+void* dev_acquire(size_t n, size_t& cap, int& device);
+// Waits for the device (as hipFree does), then keeps or frees the block.
+void dev_release(void* p, size_t cap, int device) noexcept;
+// Frees the idle blocks of the device.
+void dev_trim(int device) noexcept;
+
 // Device buffer with RAII free.
 struct DevBuf {
     void* p = nullptr;
-    size_t bytes = 0;
+    size_t bytes = 0;   // requested
+    size_t cap = 0;     // of the block
+    int device = 0;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { release(); }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) dev_release(p, cap, device);  // in-flight kernels may still use p
         p = nullptr;
-        bytes = 0;
+        bytes = cap = 0;
     }
     void alloc(size_t n) {
         if (n == bytes && p) return;
-        if (p) MSR_HIP(hipDeviceSynchronize());  // in-flight kernels may still use p
         release();
         if (n == 0) return;
-        MSR_HIP(hipMalloc(&p, n));
+        p = dev_acquire(n, cap, device);
         bytes = n;
     }
     template <class T> T* as() const { return reinterpret_cast<T*>(p); }

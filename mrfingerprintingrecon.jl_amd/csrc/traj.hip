@@ -15,6 +15,7 @@ msr_ctx::~msr_ctx() {
     for (auto& kv : twiddles64) (void)hipFree(kv.second);
     for (auto& kv : deapod) (void)hipFree(kv.second);
     for (auto& kv : deapod64) (void)hipFree(kv.second);
+    msr::dev_trim(device);
 }
 
 namespace msr {
