@@ -79,19 +79,6 @@ __global__ void kspread_points_kernel(const float* __restrict__ kc, const int* _
     }
 }
 
-// first[b] = first sorted sample of bin >= b (b <= nbins), by binary search
-__global__ void kspread_first_kernel(const int* __restrict__ sorted, int M, int nbins, int* __restrict__ first) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b > nbins) return;
-    int lo = 0, hi = M;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (sorted[mid] < b) lo = mid + 1;
-        else hi = mid;
-    }
-    first[b] = lo;
-}
-
 // vals[(t T + tile) 16 + i]: row i of a tile of 8 complex (16 real) channels:
 // channel (i / 8) 4 + i mod 4, part (i / 4) mod 2; a real basis: channel i
 __global__ void kspread_values_kernel(ValueSrc src, int np, int tiles, double* __restrict__ vals) {
@@ -265,9 +252,7 @@ void KernelSpread::build(const msr_traj* traj, const int64_t* grid_n, hipStream_
     temp.alloc(std::max<size_t>(tb, 16));
     MSR_HIP(hipcub::DeviceRadixSort::SortPairs(temp.p, tb, keys.as<int>(), sorted.as<int>(), idx.as<int>(),
                                                perm.as<int>(), (int)M, 0, bits, st));
-    hipLaunchKernelGGL(kspread_first_kernel, dim3((unsigned)(nbins / 256 + 1)), dim3(256), 0, st,
-                       sorted.as<int>(), (int)M, (int)nbins, first.as<int>());
-    MSR_CHECK_LAUNCH();
+    sorted_first(sorted.as<int>(), M, nbins, first.as<int>(), st);
     const int gw = (int)std::min<int64_t>((M * d * 8 + 255) / 256, 32768);
     if (d == 2)
         hipLaunchKernelGGL(kspread_points_kernel<2>, dim3(gw), dim3(256), 0, st, traj->kc.as<float>(),

@@ -63,8 +63,8 @@ struct PlanGeom {
 };
 
 // ------------------------------------------------------------------ sort
-__global__ void bin_count_kernel(const float* __restrict__ kc, int d, int64_t M, PlanGeom g,
-                                 int* __restrict__ counts, int* __restrict__ binid) {
+__global__ void bin_id_kernel(const float* __restrict__ kc, int d, int64_t M, PlanGeom g,
+                              int* __restrict__ binid, int* __restrict__ idx) {
     for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < M;
          j += (int64_t)gridDim.x * blockDim.x) {
         int b = 0, mul = 1;
@@ -76,51 +76,26 @@ __global__ void bin_count_kernel(const float* __restrict__ kc, int d, int64_t M,
             mul *= g.nb[a];
         }
         binid[j] = b;
-        atomicAdd(&counts[b], 1);
+        idx[j] = (int)j;
     }
 }
 
-// exclusive scan of counts into offs[0..nb], single block
-__global__ void bin_scan_kernel(const int* __restrict__ counts, int64_t nb, int* __restrict__ offs) {
-    __shared__ int s[1024];
-    __shared__ int carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int64_t base = 0; base < nb; base += 1024) {
-        const int64_t i = base + threadIdx.x;
-        const int v0 = i < nb ? counts[i] : 0;
-        s[threadIdx.x] = v0;
-        __syncthreads();
-        for (int o = 1; o < 1024; o <<= 1) {
-            int v = threadIdx.x >= o ? s[threadIdx.x - o] : 0;
-            __syncthreads();
-            s[threadIdx.x] += v;
-            __syncthreads();
-        }
-        if (i < nb) offs[i] = carry + s[threadIdx.x] - v0;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry += s[1023];
-        __syncthreads();
+__global__ void sorted_first_kernel(const int* __restrict__ sorted, int n, int nkeys, int* __restrict__ first) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b > nkeys) return;
+    int lo = 0, hi = n;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sorted[mid] < b) lo = mid + 1;
+        else hi = mid;
     }
-    if (threadIdx.x == 0) offs[nb] = carry;
+    first[b] = lo;
 }
 
-__global__ void izero_kernel(int* __restrict__ p, int64_t n) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = 0;
-}
-
-static void izero(int* p, int64_t n, hipStream_t st) {
-    int grid = (int)std::min<int64_t>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(izero_kernel, dim3(grid), dim3(256), 0, st, p, n);
+void sorted_first(const int* sorted, int64_t n, int64_t nkeys, int* first, hipStream_t st) {
+    hipLaunchKernelGGL(sorted_first_kernel, dim3((unsigned)(nkeys / 256 + 1)), dim3(256), 0, st, sorted,
+                       (int)n, (int)nkeys, first);
     MSR_CHECK_LAUNCH();
-}
-
-__global__ void iota_kernel(int* __restrict__ p, int64_t n) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = (int)i;
 }
 
 // Points sorted by tile with a stable radix sort (ties keep sample order), so
@@ -150,19 +125,15 @@ const SpreadPlan& spread_plan(const msr_traj* traj, const int64_t* n, hipStream_
         g.nb[a] = p->nb[a];
     }
     const int M = (int)traj->M;
-    DevBuf counts, binid, binsorted, idx, temp;
-    counts.alloc(sizeof(int) * p->nbins);
+    DevBuf binid, binsorted, idx, temp;
     binid.alloc(sizeof(int) * M);
     binsorted.alloc(sizeof(int) * M);
     idx.alloc(sizeof(int) * M);
     p->perm.alloc(sizeof(int) * M);
     p->offs.alloc(sizeof(int) * (p->nbins + 1));
-    izero(counts.as<int>(), p->nbins, st);
     int grid = (int)std::min<int64_t>((traj->M + 255) / 256, 8192);
-    hipLaunchKernelGGL(bin_count_kernel, dim3(grid), dim3(256), 0, st, traj->kc.as<float>(),
-                       traj->d, traj->M, g, counts.as<int>(), binid.as<int>());
-    MSR_CHECK_LAUNCH();
-    hipLaunchKernelGGL(iota_kernel, dim3(grid), dim3(256), 0, st, idx.as<int>(), traj->M);
+    hipLaunchKernelGGL(bin_id_kernel, dim3(grid), dim3(256), 0, st, traj->kc.as<float>(), traj->d,
+                       traj->M, g, binid.as<int>(), idx.as<int>());
     MSR_CHECK_LAUNCH();
     int bits = 1;
     while ((int64_t(1) << bits) < p->nbins) ++bits;
@@ -174,9 +145,7 @@ const SpreadPlan& spread_plan(const msr_traj* traj, const int64_t* n, hipStream_
     MSR_HIP(hipcub::DeviceRadixSort::SortPairs(temp.p, tbytes, binid.as<int>(),
                                                binsorted.as<int>(), idx.as<int>(),
                                                p->perm.as<int>(), M, 0, bits, st));
-    hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(1024), 0, st, counts.as<int>(), p->nbins,
-                       p->offs.as<int>());
-    MSR_CHECK_LAUNCH();
+    sorted_first(binsorted.as<int>(), M, p->nbins, p->offs.as<int>(), st);
     MSR_HIP(hipStreamSynchronize(st));  // temporaries are freed on return
     auto& ref = *p;
     traj->plans[key] = std::move(p);

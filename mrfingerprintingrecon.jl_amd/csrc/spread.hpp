@@ -22,6 +22,12 @@ constexpr int SPREAD_HALO = 4;              // cells of halo on each tile side
 // Build (or fetch from the trajectory's cache) the tile sort for grid n.
 const SpreadPlan& spread_plan(const msr_traj* traj, const int64_t* n, hipStream_t st);
 
+// first[b] = position of the first of n sorted keys that is >= b, for b <= nkeys
+// (nkeys + 1 values, keys < nkeys), by binary search: counting with atomics
+// serialises on the centre of a radial trajectory (0.3-1.6 ms per sort at
+// 512 000 samples, 4.6 ms for the 3D pairs; 7 us this way).
+void sorted_first(const int* sorted, int64_t n, int64_t nkeys, int* first, hipStream_t st);
+
 // Values of the spread channels for one point: BP or kernel-build sources.
 struct ValueSrc {
     int kind;             // 0: backprojection data, 1: basis pair products

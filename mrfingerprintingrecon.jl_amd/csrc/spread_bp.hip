@@ -106,12 +106,6 @@ __global__ void bp_emit_pairs_kernel(const int2* __restrict__ cell, const int* _
     }
 }
 
-__global__ void bp_tile_count_kernel(const int* __restrict__ keys, int64_t n, int* __restrict__ counts) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        atomicAdd(&counts[keys[i]], 1);
-}
-
 // Per pair q (point s in block t): the kernel weights of s over the block's 8
 // columns (pw[q][0..7]) and 8 rows (pw[q][8..15]), zero off the support and
 // off the grid.
@@ -162,7 +156,7 @@ void spread_streams(const msr_traj* traj, SpreadPlan& plan, hipStream_t st) {
     plan.frame_s.alloc(sizeof(int) * Mp);
     plan.jsel_s.alloc(sizeof(int64_t) * Mp);
     plan.kc_s.alloc(sizeof(float2) * Mp);
-    DevBuf npp, ppos, keys, keys_sorted, vals, temp, counts;
+    DevBuf npp, ppos, keys, keys_sorted, vals, temp, first;
     npp.alloc(sizeof(int) * (Mp + 1));
     ppos.alloc(sizeof(int) * (Mp + 1));
     const int grid = (int)std::min<int64_t>((M + 255) / 256, 8192);
@@ -221,24 +215,18 @@ void spread_streams(const msr_traj* traj, SpreadPlan& plan, hipStream_t st) {
                            (int64_t)total, g, plan.pw.as<float>());
         MSR_CHECK_LAUNCH();
     }
-    // per-tile pair counts -> work items (host)
-    counts.alloc(sizeof(int) * ntiles);
-    fill_floats(counts.p, ntiles, 0.f, st);
-    if (total > 0) {
-        const int g2 = (int)std::min<int64_t>((total + 255) / 256, 8192);
-        hipLaunchKernelGGL(bp_tile_count_kernel, dim3(g2), dim3(256), 0, st, keys_sorted.as<int>(),
-                           (int64_t)total, counts.as<int>());
-        MSR_CHECK_LAUNCH();
-    }
-    std::vector<int> hc(ntiles);
-    MSR_HIP(hipMemcpyAsync(hc.data(), counts.p, sizeof(int) * ntiles, hipMemcpyDeviceToHost, st));
+    // pairs per tile -> work items (host)
+    first.alloc(sizeof(int) * (ntiles + 1));
+    sorted_first(keys_sorted.as<int>(), total, ntiles, first.as<int>(), st);
+    std::vector<int> hf(ntiles + 1);
+    MSR_HIP(hipMemcpyAsync(hf.data(), first.p, sizeof(int) * (ntiles + 1), hipMemcpyDeviceToHost, st));
     MSR_HIP(hipStreamSynchronize(st));
     std::vector<int4> items;
     std::vector<int2> split;
     std::vector<int> split_n;
     int q = 0, slot = 0;
     for (int64_t t = 0; t < ntiles; ++t) {
-        const int cnt = hc[t];
+        const int cnt = hf[t + 1] - hf[t];
         if (cnt > ITEM_PAIRS) {
             split.push_back(make_int2((int)t, (int)items.size()));
             split_n.push_back((cnt + ITEM_PAIRS - 1) / ITEM_PAIRS);

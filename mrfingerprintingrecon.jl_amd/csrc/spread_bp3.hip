@@ -110,13 +110,6 @@ __global__ void bp3_emit_pairs_kernel(const int4* __restrict__ cell, const int* 
     }
 }
 
-__global__ void bp3_block_count_kernel(const int* __restrict__ keys, int64_t n,
-                                       int* __restrict__ counts) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        atomicAdd(&counts[keys[i]], 1);
-}
-
 // Per pair q (point s in block b): the kernel weights of s over the block's 4
 // columns (pw[q][0..3]), rows (pw[q][4..7]) and planes (pw[q][8..11]), zero off
 // the support and off the grid.
@@ -181,7 +174,7 @@ void spread_streams3(const msr_traj* traj, SpreadPlan& plan, hipStream_t st) {
     plan.frame_s.alloc(sizeof(int) * Mp);
     plan.jsel_s.alloc(sizeof(int64_t) * Mp);
     plan.r2_s.alloc(sizeof(float) * Mp);
-    DevBuf npp, ppos, keys, keys_sorted, vals, temp, counts;
+    DevBuf npp, ppos, keys, keys_sorted, vals, temp, first;
     npp.alloc(sizeof(int) * (Mp + 1));
     ppos.alloc(sizeof(int) * (Mp + 1));
     const int grid = (int)std::min<int64_t>((M + 255) / 256, 8192);
@@ -240,24 +233,18 @@ void spread_streams3(const msr_traj* traj, SpreadPlan& plan, hipStream_t st) {
                            plan.pairs.as<int>(), (int64_t)total, g, plan.pw.as<float>());
         MSR_CHECK_LAUNCH();
     }
-    // per-block pair counts -> work items (host)
-    counts.alloc(sizeof(int) * nblocks);
-    fill_floats(counts.p, nblocks, 0.f, st);
-    if (total > 0) {
-        const int g2 = (int)std::min<int64_t>((total + 255) / 256, 8192);
-        hipLaunchKernelGGL(bp3_block_count_kernel, dim3(g2), dim3(256), 0, st,
-                           keys_sorted.as<int>(), (int64_t)total, counts.as<int>());
-        MSR_CHECK_LAUNCH();
-    }
-    std::vector<int> hc(nblocks);
-    MSR_HIP(hipMemcpyAsync(hc.data(), counts.p, sizeof(int) * nblocks, hipMemcpyDeviceToHost, st));
+    // pairs per block -> work items (host)
+    first.alloc(sizeof(int) * (nblocks + 1));
+    sorted_first(keys_sorted.as<int>(), total, nblocks, first.as<int>(), st);
+    std::vector<int> hf(nblocks + 1);
+    MSR_HIP(hipMemcpyAsync(hf.data(), first.p, sizeof(int) * (nblocks + 1), hipMemcpyDeviceToHost, st));
     MSR_HIP(hipStreamSynchronize(st));
     std::vector<int4> items;
     std::vector<int2> split;
     std::vector<int> split_n;
     int q = 0, slot = 0;
     for (int64_t t = 0; t < nblocks; ++t) {
-        const int cnt = hc[t];
+        const int cnt = hf[t + 1] - hf[t];
         if (cnt > ITEM_PAIRS) {
             split.push_back(make_int2((int)t, (int)items.size()));
             split_n.push_back((cnt + ITEM_PAIRS - 1) / ITEM_PAIRS);
