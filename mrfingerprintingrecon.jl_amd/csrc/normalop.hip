@@ -124,14 +124,21 @@ void op_alloc_scratch(msr_normalop* op) {
         G = std::max(1, std::min(G, op->C));
         op->G = env_int("MSR_G", G);
         op->G = std::max(1, std::min(op->G, op->C));
-        const int64_t colblocks = 2 * op->N[0];
-        int Gb = colblocks >= 1024 ? 1 : 2;
-        op->Gb = std::max(1, std::min(env_int("MSR_GB", Gb), op->C));
         // untuned knobs: the orders measured fastest at 256^2 / 20 coils / K = 5
         // (pass A tile-fastest only with 16-byte intermediates); a tuned choice
         // for the same shape on this context replaces them
         for (int am = 0; am < 3; ++am) {
-            op->knobs[am].Gb = op->Gb;
+            // pass B's coil groups (its workgroups walk a group's coils one after
+            // another): the largest power of two up to 8 with at most 640
+            // workgroups, two to three per CU, and two groups for up to 1024
+            // columns (128 x 192, K = 8, f32: 144 / 119 / 154 / 179 us per apply
+            // with 1 / 2 / 4 / 8 groups of 256 workgroups; 64 x 64, K = 4: 45 / 33 /
+            // 28 / 26 us with groups of 32)
+            const int cb = pass_b_colblocks((int)(2 * op->N[0]), (int)(2 * ny), op->K, am != AM_F32);
+            int Gb = 2 * op->N[0] < 1024 ? 2 : 1;
+            while (Gb < 8 && cb * 2 * Gb <= 640) Gb *= 2;
+            while (Gb > op->C) Gb /= 2;
+            op->knobs[am].Gb = std::max(1, std::min(env_int("MSR_GB", Gb), op->C));
             op->knobs[am].order_a = am == AM_F64 ? 0 : 1;
             op->knobs[am].order_c = 1;
             ApplyKnobs t;
