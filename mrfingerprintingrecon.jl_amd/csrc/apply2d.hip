@@ -3,15 +3,21 @@
 // templated on the complex arithmetic type CT (float2 or double2).
 #include "apply2d.hpp"
 #include "apply2d_b.hpp"
-#include "fft.hpp"
+#include "wgfft.hpp"
 
 namespace msr {
 
 template <int NX2, class CT, class ST>
 constexpr int rowpass_block() {
+    if (wg_preferred<NX2>()) return (rows_per_tile<CT, ST>() * NX2 / WG_VALUES + 63) / 64 * 64;
     return (rows_per_tile<CT, ST>() * FFTPlan<NX2>::T) < 256
                ? rows_per_tile<CT, ST>() * FFTPlan<NX2>::T
                : 256;
+}
+
+template <int NX2, class CT, class ST>
+constexpr int rowpass_bound() {
+    return rowpass_block<NX2, CT, ST>() > 256 ? rowpass_block<NX2, CT, ST>() : 256;
 }
 
 // Workgroups are dispatched to the 8 XCDs round-robin (block b on XCD b % 8),
@@ -43,11 +49,11 @@ __device__ __forceinline__ int64_t xcd_order(int64_t lb, int64_t nblk) {
 // 0.266 ms (compact), but from 0.303 to 0.309 ms with ComplexF64 storage.
 template <int N, class ST>
 constexpr bool rowreg_first() {
-    return sizeof(ST) <= 8 && fft_plan_exact<N>() && FFTPlan<N>::R[0] % 2 == 0;
+    return !wg_preferred<N>() && sizeof(ST) <= 8 && fft_plan_exact<N>() && FFTPlan<N>::R[0] % 2 == 0;
 }
 template <int N, class ST>
 constexpr bool rowreg_last() {
-    return sizeof(ST) <= 8 && fft_plan_exact<N>() &&
+    return !wg_preferred<N>() && sizeof(ST) <= 8 && fft_plan_exact<N>() &&
            FFTPlan<N>::R[FFTPlan<N>::NST - 1] % 2 == 0;
 }
 
@@ -60,8 +66,14 @@ __device__ __forceinline__ void pass_a_body(const Apply2DArgs& a, int64_t lb) {
     constexpr int RT = rows_per_tile<CT, ST>();
     constexpr int TP = FFTPlan<NX2>::T;
     constexpr int BLK = rowpass_block<NX2, CT, ST>();
+    constexpr bool WG = wg_preferred<NX2>();
     constexpr int F = BLK / TP;              // rows transformed concurrently
-    constexpr int LD = lds_line<NX2, CT>() + 1;  // LDS row pitch (odd: transposed access)
+    // LDS row pitch (odd: transposed access)
+    constexpr int LD = WG ? wg_pitch<NX2, CT>() : lds_line<NX2, CT>() + 1;
+    auto at = [](int i) {
+        if constexpr (WG) return wg_at<NX2, CT>(i);
+        else return lds_pad<NX2, CT>(i);
+    };
     // ComplexF64 twiddles are read from the global table (L1 / L2), which frees
     // LDS for one more workgroup per CU; ComplexF32 ones from an LDS copy
     __shared__ CT s_tw_lds[sizeof(CT) == 16 ? 1 : NX2];
@@ -87,7 +99,16 @@ __device__ __forceinline__ void pass_a_body(const Apply2DArgs& a, int64_t lb) {
     const CT* bk = static_cast<const CT*>(a.b) + (size_t)k * nx * ny;
     const float2* cm = a.cmaps ? a.cmaps + (size_t)c * nx * ny : nullptr;
     const int g = tid / TP, t = tid - g * TP;
-    if constexpr (rowreg_first<NX2, ST>()) {
+    if constexpr (WG) {
+        if constexpr (sizeof(CT) != 16) __syncthreads();  // twiddles
+        wg_fft<NX2, -1, 0, 1, true, false, CT, true>(s_rows, RT, s_tw, false, false, 0,
+            [&](int l, int i) {
+                if ((FFTPlan<NX2>::R[0] % 2 && i >= NX2 / 2) || y0 + l >= ny) return cz<CT>();
+                const size_t o = (size_t)(y0 + l) * nx + i;
+                return cm ? cmul(cto<CT>(cm[o]), bk[o]) : bk[o];
+            },
+            [](int, int, int, int, CT) {});
+    } else if constexpr (rowreg_first<NX2, ST>()) {
         // each line's threads load their row (times the coil map) straight
         // into the first stage's layout, x = t + p TP + r NX2/R0 at reg[p R0 + r];
         // x < nx = NX2/2 exactly for r < R0/2, the rest is the zero padding
@@ -132,17 +153,17 @@ __device__ __forceinline__ void pass_a_body(const Apply2DArgs& a, int64_t lb) {
     for (int e = tid; e < RT * NX2; e += BLK) {
         const int yl = e % RT, qx = e / RT;
         const int y = y0 + yl;
-        if (y < ny) st_store<CT, ST>(Tk + (size_t)qx * ny + y, s_rows[yl * LD + lds_pad<NX2, CT>(qx)]);
+        if (y < ny) st_store<CT, ST>(Tk + (size_t)qx * ny + y, s_rows[yl * LD + at(qx)]);
     }
 }
 
 template <int NX2, class CT, class ST>
-__global__ void __launch_bounds__(256) pass_a_2d(Apply2DArgs a) {
+__global__ void __launch_bounds__((rowpass_bound<NX2, CT, ST>())) pass_a_2d(Apply2DArgs a) {
     pass_a_body<NX2, CT, ST>(a, blockIdx.x);
 }
 
 template <int NX2, class CT, class ST>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__((rowpass_bound<NX2, CT, ST>()))
 pass_a_2d_batch(const Apply2DArgs* __restrict__ jobs, const int* __restrict__ pre, int nj) {
     const int j = batch_job(pre, nj, blockIdx.x);
     pass_a_body<NX2, CT, ST>(jobs[j], (int64_t)blockIdx.x - pre[j]);
@@ -156,15 +177,17 @@ __device__ __forceinline__ void pass_c_body(const Apply2DArgs& a, int64_t lb) {
     constexpr int RT = rows_per_tile<CT, ST>();
     constexpr int TP = FFTPlan<NX2>::T;
     constexpr int BLK = rowpass_block<NX2, CT, ST>();
+    constexpr bool WG = wg_preferred<NX2>();
     constexpr int F = BLK / TP;
-    constexpr int LD = lds_line<NX2, CT>() + 1;
+    constexpr int LD = WG ? wg_pitch<NX2, CT>() : lds_line<NX2, CT>() + 1;
     constexpr int NXC = NX2 / 2;                 // = nx
     constexpr bool LASTREG = rowreg_last<NX2, ST>();
     constexpr int RL = FFTPlan<NX2>::R[FFTPlan<NX2>::NST - 1], NBL = NX2 / RL;
     constexpr int HALF = NX2 / TP / 2;           // cropped outputs per line and thread
     // accumulators: per thread EA elements of the tile (LDS crop), or HALF per
     // line it transforms (register crop)
-    constexpr int EA = LASTREG ? (RT / F) * HALF : (RT * NXC + BLK - 1) / BLK;
+    constexpr int PERL = wg_per(RL);              // WG: the last stage's outputs
+    constexpr int EA = WG ? PERL * RL : LASTREG ? (RT / F) * HALF : (RT * NXC + BLK - 1) / BLK;
     // ComplexF64 twiddles are read from the global table (L1 / L2), which frees
     // LDS for one more workgroup per CU; ComplexF32 ones from an LDS copy
     __shared__ CT s_tw_lds[sizeof(CT) == 16 ? 1 : NX2];
@@ -191,6 +214,38 @@ __device__ __forceinline__ void pass_c_body(const Apply2DArgs& a, int64_t lb) {
     CT acc[EA];
 #pragma unroll
     for (int i = 0; i < EA; ++i) acc[i] = cz<CT>();
+    CT* pk = static_cast<CT*>(a.partial) + ((size_t)grp * K + k) * nx * ny;
+    if constexpr (WG) {
+        if constexpr (sizeof(CT) != 16) __syncthreads();  // twiddles
+        constexpr int SH = RT == 4 ? 2 : 3;
+        static_assert(RT == 1 << SH);
+        for (int c = c0; c < c1; ++c) {
+            const ST* Tk = static_cast<const ST*>(a.T) + ((size_t)c * K + k) * NX2 * ny + y0;
+            const float2* cm = a.cmaps ? a.cmaps + (size_t)c * nx * ny : nullptr;
+            wg_fft<NX2, +1, 0, 1, true, true, CT>(s_rows, RT, s_tw, true, false, SH,
+                [&](int l, int q) {
+                    return y0 + l < ny ? st_load<CT, ST>(Tk + (size_t)q * ny + l) : cz<CT>();
+                },
+                [&](int p, int r, int l, int i, CT v) {
+                    if (i < NXC && y0 + l < ny) {
+                        CT& ac = acc[p * RL + r];
+                        if (cm) cfmac(ac, cto<CT>(cm[(size_t)(y0 + l) * nx + i]), v);
+                        else ac = cadd(ac, v);
+                    }
+                });
+            __syncthreads();  // the rows are read before the next coil's are written
+        }
+#pragma unroll
+        for (int p = 0; p < PERL; ++p) {
+            const int m = tid + p * BLK;
+            if (m >= RT * NBL) continue;
+            const int l = m / NBL, j = m - l * NBL;
+#pragma unroll
+            for (int r = 0; r < RL; ++r)
+                if (j + r * NBL < NXC && y0 + l < ny) pk[(size_t)(y0 + l) * nx + j + r * NBL] = acc[p * RL + r];
+        }
+        return;
+    }
     const int g = tid / TP, t = tid - g * TP;
     // the tile's rows of one coil, NLE elements per thread, prefetched into
     // registers one coil ahead
@@ -256,7 +311,6 @@ __device__ __forceinline__ void pass_c_body(const Apply2DArgs& a, int64_t lb) {
         }
         __syncthreads();
     }
-    CT* pk = static_cast<CT*>(a.partial) + ((size_t)grp * K + k) * nx * ny;
     if constexpr (LASTREG) {
 #pragma unroll
         for (int r0 = 0; r0 < RT; r0 += F) {
@@ -283,12 +337,12 @@ __device__ __forceinline__ void pass_c_body(const Apply2DArgs& a, int64_t lb) {
 }
 
 template <int NX2, class CT, class ST>
-__global__ void __launch_bounds__(256) pass_c_2d(Apply2DArgs a) {
+__global__ void __launch_bounds__((rowpass_bound<NX2, CT, ST>())) pass_c_2d(Apply2DArgs a) {
     pass_c_body<NX2, CT, ST>(a, blockIdx.x);
 }
 
 template <int NX2, class CT, class ST>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__((rowpass_bound<NX2, CT, ST>()))
 pass_c_2d_batch(const Apply2DArgs* __restrict__ jobs, const int* __restrict__ pre, int nj) {
     const int j = batch_job(pre, nj, blockIdx.x);
     pass_c_body<NX2, CT, ST>(jobs[j], (int64_t)blockIdx.x - pre[j]);

@@ -4,7 +4,7 @@
 #pragma once
 
 #include "apply2d.hpp"
-#include "fft.hpp"
+#include "wgfft.hpp"
 
 namespace msr {
 #ifndef PB_WAVES
@@ -84,7 +84,12 @@ __device__ __forceinline__ void pass_b_body(const Apply2DArgs& a, int64_t lb) {
     // the swizzled LDS layout up to K = 5 (above, its address arithmetic
     // makes the pass spill)
     constexpr bool SWZ = lds_swizzled<NY2, CT>() && K <= 5;
-    constexpr int LL = lds_line<NY2, CT, SWZ>();
+    constexpr bool WG = wg_preferred<NY2>();
+    constexpr int LL = WG ? wg_pitch<NY2, CT>() : lds_line<NY2, CT, SWZ>();
+    auto at = [](int i) {
+        if constexpr (WG) return wg_at<NY2, CT>(i);
+        else return lds_pad<NY2, CT, SWZ>(i);
+    };
     // ComplexF64 twiddles are read from the global table (L1 / L2), which frees
     // LDS for one more workgroup per CU; ComplexF32 ones from an LDS copy
     __shared__ CT s_tw_lds[sizeof(CT) == 16 ? 1 : NY2];
@@ -154,23 +159,36 @@ __device__ __forceinline__ void pass_b_body(const Apply2DArgs& a, int64_t lb) {
                 }
             }
     };
-    if (PREFETCH && c0 < c1) prefetch(c0);
+    if constexpr (!WG && PREFETCH)
+        if (c0 < c1) prefetch(c0);
     __syncthreads();  // twiddles
     for (int c = c0; c < c1; ++c) {
-        CT xr[NR];
-        if constexpr (!PREFETCH) prefetch(c);
+        CT xr[WG ? 1 : NR];
+        ST* Tc = T + (size_t)c * K * nx2 * ny + (size_t)qx0 * ny;
+        if constexpr (WG) {
+            // line l = column K + coefficient
+            wg_fft<NY2, -1, 0, 1, true, false, CT, true>(s_buf, WC * K, s_tw, false, false, 0,
+                [&](int l, int i) {
+                    const int w = l / K, k = l - w * K;
+                    if (FFTPlan<NY2>::R[0] % 2 && i >= NY2 / 2) return cz<CT>();
+                    return qx0 + w < nx2 ? st_load<CT, ST>(Tc + ((size_t)k * nx2 + w) * ny + i) : cz<CT>();
+                },
+                [](int, int, int, int, CT) {});
+        } else {
+            if constexpr (!PREFETCH) prefetch(c);
 #pragma unroll
-        for (int e = 0; e < NR; ++e) xr[e] = pre[e];
-        if (PREFETCH && c + 1 < c1) prefetch(c + 1);  // in flight during this coil's transforms
-        if (fft_thread) fft_wave<NY2, -1, true, false, CT, SWZ>(line, s_tw, t, true, xr);
-        __syncthreads();
+            for (int e = 0; e < NR; ++e) xr[e] = pre[e];
+            if (PREFETCH && c + 1 < c1) prefetch(c + 1);  // in flight during this coil's transforms
+            if (fft_thread) fft_wave<NY2, -1, true, false, CT, SWZ>(line, s_tw, t, true, xr);
+            __syncthreads();
+        }
         // per-voxel Hermitian (or real symmetric) K x K multiply
 #pragma unroll
         for (int e = 0; e < EV; ++e) {
             const int v = tid + e * BLK;
             if (v < NV) {
                 const int wc = v / NY2, qy = v - wc * NY2;
-                CT* col = s_buf + (size_t)wc * K * LL + lds_pad<NY2, CT, SWZ>(qy);
+                CT* col = s_buf + (size_t)wc * K * LL + at(qy);
                 CT in[K], acc[K];
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
@@ -189,7 +207,17 @@ __device__ __forceinline__ void pass_b_body(const Apply2DArgs& a, int64_t lb) {
             }
         }
         __syncthreads();
-        if (fft_thread) {
+        if constexpr (WG) {
+            wg_fft<NY2, +1, 0, 1, false, true, CT, true>(s_buf, WC * K, s_tw, false, false, 0,
+                [](int, int) { return cz<CT>(); },
+                [&](int, int, int l, int i, CT v) {
+                    const int w = l / K, k = l - w * K;
+                    if (FFTPlan<NY2>::R[FFTPlan<NY2>::NST - 1] % 2 && i >= NY2 / 2) return;
+                    if (qx0 + w < nx2)
+                        st_store<CT, ST>(Tc + ((size_t)k * nx2 + w) * ny + i, v);
+                });
+            __syncthreads();  // the lines are read before the next coil's are written
+        } else if (fft_thread) {
             ST* dst = T + (((size_t)c * K + kl) * nx2 + qx0 + wcl) * ny;
             constexpr int RL = FFTPlan<NY2>::R[FFTPlan<NY2>::NST - 1], NBL = NY2 / RL;
             if constexpr (PB_CROPREG && RL % 2 == 0 && sizeof(ST) <= 8) {

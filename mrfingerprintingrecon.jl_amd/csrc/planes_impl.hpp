@@ -1,26 +1,17 @@
 // Kernels of the fused line passes (see planes.hpp), instantiated per length
-// by the planes_p*.hip translation units.
-//
-// The lines of a workgroup are transformed by all its threads together: a
-// stage's butterflies, over all lines, are dealt out to the threads, at most 8
-// values (10 in radix 5, 9 in radix 3) per thread, whatever the length's
-// factors, and stages are separated by workgroup barriers.  A transform by a
-// few threads per line (fft_lds) holds up to 40 values per thread at these
-// lengths: the multiply then took 148-256 VGPRs, one workgroup per CU, and
-// 443 us at 240 x 300 / 12 coils / K = 6 in ComplexF64.  The first stage takes
-// its inputs from global memory and the last one hands its outputs over in
-// registers, so a line makes one LDS round trip less at either end.
+// by the planes_p*.hip translation units.  The lines of a workgroup are
+// transformed by all its threads together (wgfft.hpp): with a few threads per
+// line (fft_lds) the multiply took 148-256 VGPRs, one workgroup per CU, and
+// 443 us at 240 x 300 / 12 coils / K = 6 in ComplexF64 instead of 228.
 #pragma once
 
-#include "fft.hpp"
 #include "planes.hpp"
+#include "wgfft.hpp"
 
 namespace msr {
 
 constexpr int PLANE_KMAX = 8;        // coefficients held in registers by the multiply
-constexpr int PLANE_VALUES = 8;      // values per thread in a transform
 constexpr int PLANE_MAX_ROW = 1024;  // longest row FFT (threads of a row tile)
-constexpr int PLANE_MAX_LINE = 2048;
 
 // Workgroup i runs on XCD i mod 8: consecutive logical blocks on one XCD when
 // the count divides by 8, so neighbours share their L2's lines.
@@ -28,108 +19,19 @@ __device__ __forceinline__ int64_t plane_xcd(int64_t b, int64_t n) {
     return n % 8 ? b : (b % 8) * (n / 8) + b / 8;
 }
 
-// butterflies per thread of a radix-R stage
-constexpr int plane_per(int R) { return (PLANE_VALUES + R - 1) / R; }
-
-// One stage of nl lines of NF by the whole workgroup (blockDim.x * 8 >= nl NF):
-// in(m, p, v) fetches the R inputs of butterfly m, the thread's p-th, and
-// out(m, p, v) transforms and hands them over.  SYNC: a barrier between the two
-// (both in the same LDS lines).
-template <int NF, int R, int NS, int DIR, bool SYNC, class CT, class IN, class OUT>
-__device__ __forceinline__ void plane_stage(int nl, const CT* tw, IN&& in, OUT&& out) {
-    constexpr int NB = NF / R, PER = plane_per(R);
-    CT v[PER][R];
-#pragma unroll
-    for (int p = 0; p < PER; ++p) {
-        const int m = threadIdx.x + p * blockDim.x;
-        if (m < nl * NB) in(m, p, v[p]);
-    }
-    if constexpr (SYNC) __syncthreads();
-#pragma unroll
-    for (int p = 0; p < PER; ++p) {
-        const int m = threadIdx.x + p * blockDim.x;
-        if (m < nl * NB) out(m, p, v[p]);
-    }
-}
-
-// LDS place of element i of a line, and the pitch of the lines: the swizzled
-// layout of fft.hpp for ComplexF64 from 64 points on, its padding otherwise
-template <int NF, class CT> constexpr bool plane_swizzled() { return sizeof(CT) == 16 && NF >= 64; }
-template <int NF, class CT>
-__device__ __forceinline__ int plane_at(int i) { return lds_pad<NF, CT, plane_swizzled<NF, CT>()>(i); }
-template <int NF, class CT>
-constexpr int plane_pitch() { return lds_line<NF, CT, plane_swizzled<NF, CT>()>() + 1; }
-
-// Where butterfly m of a stage works: line l, butterfly j of the line.  Lines
-// that are neighbours in memory (2^sh of them per plane k, line k 2^sh + w) may
-// be dealt out line first, so that consecutive threads touch neighbours.
-struct PlaneSpot {
-    int l, j;
-};
-template <int NB>
-__device__ __forceinline__ PlaneSpot plane_spot(int m, bool line_first, int sh) {
-    if (!line_first) {
-        const int l = m / NB;
-        return {l, m - l * NB};
-    }
-    const int w = m & ((1 << sh) - 1), r = m >> sh, k = r / NB;
-    return {(k << sh) + w, r - k * NB};
-}
-
-// Transform of nl lines, element i of line l at s[l * LP + plane_at(i)]:
-// FIRST: get(l, i) supplies the first stage's inputs (dealt out line first if
-// lf_in), else they are in LDS; LAST: put(p, r, l, i, value) takes the last
-// stage's outputs (line first if lf_out), value p R + r of the thread, else
-// they go to LDS.  Ends with a barrier (LDS free, or the result visible) unless
-// LAST, where the caller places it before the LDS lines are written again.
-
-template <int NF, int DIR, int S, int NS, bool FIRST, bool LAST, class CT, class GET, class PUT>
-__device__ __forceinline__ void plane_fft(CT* s, int nl, const CT* tw, bool lf_in, bool lf_out, int sh,
-                                          GET&& get, PUT&& put) {
-    using Pl = FFTPlan<NF>;
-    if constexpr (S < Pl::NST) {
-        constexpr int R = Pl::R[S], NB = NF / R, LP = plane_pitch<NF, CT>();
-        constexpr bool GIN = FIRST && S == 0, POUT = LAST && S == Pl::NST - 1;
-        plane_stage<NF, R, NS, DIR, !GIN && !POUT, CT>(
-            nl, tw,
-            [&](int m, int, CT* v) {
-                const PlaneSpot q = plane_spot<NB>(m, (GIN && lf_in) || (POUT && lf_out), sh);
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    if constexpr (GIN) v[r] = get(q.l, q.j + r * NB);
-                    else v[r] = s[q.l * LP + plane_at<NF, CT>(q.j + r * NB)];
-                }
-            },
-            [&](int m, int p, CT* v) {
-                const PlaneSpot q = plane_spot<NB>(m, (GIN && lf_in) || (POUT && lf_out), sh);
-                const int k = q.j % NS;
-                stage_twiddle<NF, R, NS, DIR>(v, tw, k);
-                Butterfly<R, DIR>::run(v);
-                const int base = (q.j - k) * R + k;
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    if constexpr (POUT) put(p, r, q.l, base + r * NS, v[r]);
-                    else s[q.l * LP + plane_at<NF, CT>(base + r * NS)] = v[r];
-                }
-            });
-        if constexpr (!POUT) __syncthreads();
-        plane_fft<NF, DIR, S + 1, NS * R, FIRST, LAST, CT>(s, nl, tw, lf_in, lf_out, sh, get, put);
-    }
-}
-
 // rows per tile: 64-byte pieces of neighbouring rows, more for short lines
 // (at least 128 threads)
 template <int NF, class CT>
 constexpr int plane_rows() {
     int f = sizeof(CT) == 16 ? 4 : 8;
-    while (f < 32 && f * NF < 128 * PLANE_VALUES) f *= 2;
-    while (f > 1 && f * NF > 1024 * PLANE_VALUES) f /= 2;
+    while (f < 32 && f * NF < 128 * WG_VALUES) f *= 2;
+    while (f > 1 && f * NF > 1024 * WG_VALUES) f /= 2;
     return f;
 }
 constexpr int plane_shift(int f) { return f <= 1 ? 0 : 1 + plane_shift(f / 2); }
 template <int NF, class CT>
 constexpr int plane_row_block() {
-    return ((plane_rows<NF, CT>() * NF + PLANE_VALUES - 1) / PLANE_VALUES + 63) / 64 * 64;
+    return ((plane_rows<NF, CT>() * NF + WG_VALUES - 1) / WG_VALUES + 63) / 64 * 64;
 }
 
 // ---------------------------------------------------------------- expand
@@ -140,7 +42,7 @@ __global__ void __launch_bounds__((plane_row_block<NF, CT>()))
 plane_expand_kernel(PlanePass p, const CT* __restrict__ tw) {
     if (p.skip && *p.skip) return;
     constexpr int F = plane_rows<NF, CT>(), SH = plane_shift(F), BLK = plane_row_block<NF, CT>();
-    constexpr int LP = plane_pitch<NF, CT>();
+    constexpr int LP = wg_pitch<NF, CT>();
     __shared__ CT s[F * LP];
     const int64_t tiles = (p.nrows + F - 1) / F;
     const int64_t lb = plane_xcd(blockIdx.x, tiles * p.K * p.nc);
@@ -156,14 +58,14 @@ plane_expand_kernel(PlanePass p, const CT* __restrict__ tw) {
         return cm ? cmul(cto<CT>(cm[l * len + i]), v) : v;
     };
     if (p.qs == 1) {  // rows stay rows: straight from the last stage
-        plane_fft<NF, -1, 0, 1, true, true, CT>(s, F, tw, false, false, SH, get,
+        wg_fft<NF, -1, 0, 1, true, true, CT>(s, F, tw, false, false, SH, get,
             [&](int, int, int l, int q, CT v) { if (l < nr) T[l * p.rs + q] = v; });
         return;
     }
-    plane_fft<NF, -1, 0, 1, true, false, CT>(s, F, tw, false, false, SH, get, [](int, int, int, int, CT) {});
+    wg_fft<NF, -1, 0, 1, true, false, CT>(s, F, tw, false, false, SH, get, [](int, int, int, int, CT) {});
     for (int e = threadIdx.x; e < F * NF; e += BLK) {
         const int q = e >> SH, l = e & (F - 1);
-        if (l < nr) T[l * p.rs + q * p.qs] = s[l * LP + plane_at<NF, CT>(q)];
+        if (l < nr) T[l * p.rs + q * p.qs] = s[l * LP + wg_at<NF, CT>(q)];
     }
 }
 
@@ -175,8 +77,8 @@ __global__ void __launch_bounds__((plane_row_block<NF, CT>()))
 plane_combine_kernel(PlanePass p, const CT* __restrict__ tw) {
     if (p.skip && *p.skip) return;
     constexpr int F = plane_rows<NF, CT>(), SH = plane_shift(F);
-    constexpr int LP = plane_pitch<NF, CT>();
-    constexpr int RL = FFTPlan<NF>::R[FFTPlan<NF>::NST - 1], PER = plane_per(RL), NBL = NF / RL;
+    constexpr int LP = wg_pitch<NF, CT>();
+    constexpr int RL = FFTPlan<NF>::R[FFTPlan<NF>::NST - 1], PER = wg_per(RL), NBL = NF / RL;
     __shared__ CT s[F * LP];
     const int64_t tiles = (p.nrows + F - 1) / F;
     const int64_t lb = plane_xcd(blockIdx.x, tiles * p.K * p.G);
@@ -193,7 +95,7 @@ plane_combine_kernel(PlanePass p, const CT* __restrict__ tw) {
             const int m = threadIdx.x + q * blockDim.x;
             if (m >= F * NBL) continue;
             // (one stage alone is dealt out as its inputs are)
-            const PlaneSpot w = plane_spot<NBL>(m, FFTPlan<NF>::NST == 1 && p.qs != 1, SH);
+            const WgSpot w = wg_spot<NBL>(m, FFTPlan<NF>::NST == 1 && p.qs != 1, SH);
 #pragma unroll
             for (int r = 0; r < RL; ++r)
                 if (w.j + r * NBL < len && w.l < nr) visit(q * RL + r, w.l * len + w.j + r * NBL);
@@ -205,7 +107,7 @@ plane_combine_kernel(PlanePass p, const CT* __restrict__ tw) {
     for (int c = c0; c < c1; ++c) {
         const CT* T = static_cast<const CT*>(p.T) + ((int64_t)c * p.K + k) * p.plane + r0 * p.rs;
         const float2* cm = p.cmaps ? p.cmaps + ((int64_t)c * p.nrows + r0) * len : nullptr;
-        plane_fft<NF, +1, 0, 1, true, true, CT>(s, F, tw, p.qs != 1, false, SH,
+        wg_fft<NF, +1, 0, 1, true, true, CT>(s, F, tw, p.qs != 1, false, SH,
             [&](int l, int q) { return l < nr ? T[l * p.rs + q * p.qs] : cz<CT>(); },
             [&](int q, int r, int l, int i, CT v) {
                 if (i < len && l < nr) {
@@ -282,7 +184,7 @@ template <int NF, class CT>
 __global__ void __launch_bounds__(1024)
 plane_multiply_kernel(PlanePass p, const CT* __restrict__ tw, int wcs) {
     if (p.skip && *p.skip) return;
-    constexpr int LP = plane_pitch<NF, CT>();
+    constexpr int LP = wg_pitch<NF, CT>();
     extern __shared__ double2 plane_lds[];
     CT* s = reinterpret_cast<CT*>(plane_lds);
     const int K = p.K, NL = K << wcs, len = p.len;
@@ -296,7 +198,7 @@ plane_multiply_kernel(PlanePass p, const CT* __restrict__ tw, int wcs) {
     const bool lf = p.es != 1;
     const int wm = (1 << wcs) - 1;
     // line l = k 2^wcs + w; a thread stores what its own block alone has read
-    plane_fft<NF, -1, 0, 1, true, false, CT>(s, NL, tw, lf, false, wcs,
+    wg_fft<NF, -1, 0, 1, true, false, CT>(s, NL, tw, lf, false, wcs,
         [&](int l, int i) {
             const int w = l & wm;
             return i < len && w < ncol ? T[(l >> wcs) * p.plane + w * p.cs + i * p.es] : cz<CT>();
@@ -306,7 +208,7 @@ plane_multiply_kernel(PlanePass p, const CT* __restrict__ tw, int wcs) {
         for (int v = threadIdx.x; v < (NF << wcs); v += blockDim.x) {
             const int w = v / NF, i = v - w * NF;
             if (w < ncol)
-                plane_cell<NF, FULL>(lam + (col0 + w) * P * NF + i, K, s + w * LP + plane_at<NF, CT>(i), LP << wcs);
+                plane_cell<NF, FULL>(lam + (col0 + w) * P * NF + i, K, s + w * LP + wg_at<NF, CT>(i), LP << wcs);
         }
     };
     if (p.lam_full) {
@@ -317,7 +219,7 @@ plane_multiply_kernel(PlanePass p, const CT* __restrict__ tw, int wcs) {
         else multiply.template operator()<false>(static_cast<const float2*>(p.lam));
     }
     __syncthreads();
-    plane_fft<NF, +1, 0, 1, false, true, CT>(s, NL, tw, false, lf, wcs,
+    wg_fft<NF, +1, 0, 1, false, true, CT>(s, NL, tw, false, lf, wcs,
         [](int, int) { return cz<CT>(); },
         [&](int, int, int l, int i, CT v) {
             const int w = l & wm;
@@ -340,7 +242,7 @@ template <int NF>
 __global__ void __launch_bounds__((plane_row_block<NF, float2>()))
 plane_place_kernel(PlanePass p, const float2* __restrict__ tw) {
     constexpr int F = plane_rows<NF, float2>(), SH = plane_shift(F), BLK = plane_row_block<NF, float2>();
-    constexpr int LP = plane_pitch<NF, float2>();
+    constexpr int LP = wg_pitch<NF, float2>();
     __shared__ float2 s[F * LP];
     const int64_t tiles = (p.nrows + F - 1) / F;
     const int64_t lb = plane_xcd(blockIdx.x, tiles * p.K * p.nc);
@@ -350,7 +252,7 @@ plane_place_kernel(PlanePass p, const float2* __restrict__ tw) {
     const float2* b = static_cast<const float2*>(p.b) + ((int64_t)k * p.nrows + r0) * len;
     const float2* cm = p.cmaps ? p.cmaps + ((int64_t)c * p.nrows + r0) * len : nullptr;
     float2* T = static_cast<float2*>(p.T) + ((int64_t)k * p.nc + c) * p.plane + r0;
-    plane_fft<NF, -1, 0, 1, true, false, float2>(s, F, tw, false, false, SH,
+    wg_fft<NF, -1, 0, 1, true, false, float2>(s, F, tw, false, false, SH,
         [&](int l, int q) {
             const int i = plane_centred<NF>(q, len);
             if (i >= len || l >= nr) return make_float2(0.f, 0.f);
@@ -360,7 +262,7 @@ plane_place_kernel(PlanePass p, const float2* __restrict__ tw) {
         [](int, int, int, int, float2) {});
     for (int e = threadIdx.x; e < F * NF; e += BLK) {
         const int q = e >> SH, l = e & (F - 1);
-        if (l < nr) T[l + (int64_t)q * p.nrows] = s[l * LP + plane_at<NF, float2>(q)];
+        if (l < nr) T[l + (int64_t)q * p.nrows] = s[l * LP + wg_at<NF, float2>(q)];
     }
 }
 
@@ -368,14 +270,14 @@ plane_place_kernel(PlanePass p, const float2* __restrict__ tw) {
 // transformed, written with the coils side by side.
 template <int NF>
 __global__ void __launch_bounds__(1024) plane_coils_kernel(PlanePass p, const float2* __restrict__ tw) {
-    constexpr int F = PLANE_COIL_GROUP, LP = plane_pitch<NF, float2>();
+    constexpr int F = PLANE_COIL_GROUP, LP = wg_pitch<NF, float2>();
     __shared__ float2 s[F * LP];
     const int CB = (p.nc + F - 1) / F, len = p.len;
     const int64_t lb = plane_xcd(blockIdx.x, p.ncols * CB * p.K);
     const int64_t col = lb % p.ncols, g = lb / p.ncols;  // g = k CB + coil group
     const int k = (int)(g / CB), c0 = (int)(g % CB) * F;
     const float2* T = static_cast<const float2*>(p.T) + ((int64_t)k * p.nc + c0) * p.plane + col * len;
-    plane_fft<NF, -1, 0, 1, true, false, float2>(s, F, tw, false, false, 3,
+    wg_fft<NF, -1, 0, 1, true, false, float2>(s, F, tw, false, false, 3,
         [&](int l, int q) {
             const int i = plane_centred<NF>(q, len);
             if (i >= len || c0 + l >= p.nc) return make_float2(0.f, 0.f);
@@ -384,7 +286,7 @@ __global__ void __launch_bounds__(1024) plane_coils_kernel(PlanePass p, const fl
         [](int, int, int, int, float2) {});
     float2* out = p.out + (g * p.ncols + col) * NF * F;
     for (int e = threadIdx.x; e < F * NF; e += blockDim.x)
-        out[e] = s[(e & (F - 1)) * LP + plane_at<NF, float2>(e / F)];
+        out[e] = s[(e & (F - 1)) * LP + wg_at<NF, float2>(e / F)];
 }
 
 // ---------------------------------------------------------------- launch
@@ -403,7 +305,7 @@ void launch_plane_n(int which, const PlanePass& p, const CT* tw, hipStream_t st)
                 hipLaunchKernelGGL((plane_place_kernel<NF>), dim3(plane_grid(tiles * p.K * p.nc)), dim3(BLK),
                                    0, st, p, tw);
             } else {
-                constexpr int BLK = (PLANE_COIL_GROUP * NF + PLANE_VALUES - 1) / PLANE_VALUES;
+                constexpr int BLK = (PLANE_COIL_GROUP * NF + WG_VALUES - 1) / WG_VALUES;
                 hipLaunchKernelGGL((plane_coils_kernel<NF>),
                                    dim3(plane_grid(p.ncols * ceil_div(p.nc, PLANE_COIL_GROUP) * p.K)),
                                    dim3((BLK + 63) / 64 * 64), 0, st, p, tw);
@@ -417,8 +319,8 @@ void launch_plane_n(int which, const PlanePass& p, const CT* tw, hipStream_t st)
         // columns per block: strided ones 64 bytes of neighbours, contiguous
         // ones up to 256 threads; fewer while the block would leave room for
         // one block per CU only, or exceed 1024 threads
-        auto bytes = [&](int w) { return sizeof(CT) * ((size_t)p.K << w) * plane_pitch<NF, CT>(); };
-        auto threads = [&](int w) { return ((p.K << w) * NF + PLANE_VALUES - 1) / PLANE_VALUES; };
+        auto bytes = [&](int w) { return sizeof(CT) * ((size_t)p.K << w) * wg_pitch<NF, CT>(); };
+        auto threads = [&](int w) { return ((p.K << w) * NF + WG_VALUES - 1) / WG_VALUES; };
         int wcs = sizeof(CT) == 16 ? 2 : 3;
         if (p.es == 1)
             for (wcs = 0; threads(wcs + 1) <= 256 && (int64_t)1 << wcs < p.ncols; ++wcs) {}
