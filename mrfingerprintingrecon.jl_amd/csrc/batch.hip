@@ -339,10 +339,10 @@ static void iterate_seq(msr_batch* bt, BatchTables& T, int niter, int am, hipStr
     CgJob<VT, AT>* cj = dev_cgjobs<VT, AT>(bt, T);
     const int* vp = dev_vpre(bt, T);
     for (int it = 0; it < niter; ++it) {
-        launch_cg_u_batch<VT, AT>(cj, vp, nj, bt->vblocks, st);
+        launch_cg_u_batch<VT, AT>(cj, vp, nj, bt->vblocks, it > 0, st);
         batch_passes(bt, T, use, st);
         launch_cg_reduce_dot_batch<VT, AT>(cj, vp, nj, bt->vblocks, st);
-        launch_cg_xr_batch<VT, AT>(cj, vp, nj, bt->vblocks, st);
+        launch_cg_xr_batch<VT, AT>(cj, vp, nj, bt->vblocks, it + 1 == niter, st);
     }
 }
 

@@ -126,7 +126,9 @@ struct CgScalars {
     double res, prev, tol;
     double alpha_re, alpha_im;
     double dot_re, dot_im;
-    int iter, done, maxiter, pad;
+    int iter, done, maxiter;
+    int pending;        // res_new is the residual of an iteration not counted yet
+    double res_new;
 };
 
 }  // namespace msr

@@ -509,12 +509,12 @@ __global__ void f32_to_f64_kernel(const float2* __restrict__ a, double2* __restr
 // kernels skip once done is set)
 template <class VT, class AT>
 static void cg_iteration(msr_normalop* op, const CgVecs<VT, AT>& v, CgScalars* S, double* part,
-                         int am, hipStream_t st) {
+                         int am, bool first, bool last, hipStream_t st) {
     const int64_t n = op->V * op->K;
-    launch_cg_u(v, n, S, st);
+    launch_cg_u(v, n, part, S, !first, st);
     op_passes(op, v.ua, am, st, &S->done);
     launch_cg_reduce_dot(op->partial.as<AT>(), op->G, n, v, op_scale(op), part, S, st, false);
-    launch_cg_xr_step(v, n, part, S, st);
+    launch_cg_xr_step(v, n, part, S, last, st);
 }
 
 // c = A x0 in the apply precision
@@ -561,7 +561,7 @@ static void cg_run(msr_normalop* op, float2* x, const float2* b, int maxiter, do
     const int am = apply_mode(prec);
     if (mode == MSR_CG_DEVICE) {
         cg_prologue(op, v, S, part, x, b, maxiter, reltol, abstol, initially_zero, am, st);
-        for (int it = 0; it < maxiter; ++it) cg_iteration(op, v, S, part, am, st);
+        for (int it = 0; it < maxiter; ++it) cg_iteration(op, v, S, part, am, it == 0, it + 1 == maxiter, st);
         cg_epilogue(op, v, x, st);
     } else if (mode == MSR_CG_GRAPH) {
         // the captured kernels hold the buffer addresses: they are part of the
@@ -583,7 +583,7 @@ static void cg_run(msr_normalop* op, float2* x, const float2* b, int maxiter, do
             MSR_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             try {
                 cg_prologue(op, v, S, part, x, b, maxiter, reltol, abstol, initially_zero, am, st);
-                for (int it = 0; it < maxiter; ++it) cg_iteration(op, v, S, part, am, st);
+                for (int it = 0; it < maxiter; ++it) cg_iteration(op, v, S, part, am, it == 0, it + 1 == maxiter, st);
                 cg_epilogue(op, v, x, st);
             } catch (...) {
                 (void)hipStreamEndCapture(st, &g);
@@ -617,7 +617,7 @@ static void cg_run(msr_normalop* op, float2* x, const float2* b, int maxiter, do
                 MSR_HIP(hipMemcpyAsync(&hs, S, sizeof(CgScalars), hipMemcpyDeviceToHost, st));
                 MSR_HIP(hipStreamSynchronize(st));
                 if (hs.done) break;
-                launch_cg_u(v, n, S, st);
+                launch_cg_u(v, n, part, S, false, st);
                 if (op->cart)
                     op_apply(op, v.c, v.ua, make_float2(1.f, 0.f), make_float2(0.f, 0.f), true, st);
                 else
@@ -731,7 +731,7 @@ static void cg_noalloc_run(msr_normalop* op, unsigned char* base, float2* x, con
     // (r, u, x and the scalars by cg_start; c, part by each iteration), so
     // nothing carried over from an earlier call is used
     cg_prologue(op, v, S, part, x, b, maxiter, reltol, abstol, initially_zero, am, st);
-    for (int it = 0; it < maxiter; ++it) cg_iteration(op, v, S, part, am, st);
+    for (int it = 0; it < maxiter; ++it) cg_iteration(op, v, S, part, am, it == 0, it + 1 == maxiter, st);
     cg_epilogue(op, v, x, st);
     *S_out = S;
 }

@@ -151,16 +151,46 @@ __device__ __forceinline__ void cg_start_finish_body(const double* __restrict__ 
     S->iter = 0;
     S->maxiter = maxiter;
     S->alpha_re = S->alpha_im = 0.0;
+    S->pending = 0;
     S->done = (maxiter <= 0 || res <= S->tol) ? 1 : 0;
 }
 
+// u = r + beta u.  With rpart, the finish of the iteration before is folded in:
+// every block sums its nb residual partials (as cg_iter_finish_body: one
+// wavefront, fixed order, the same value in each), and block 0 leaves the new
+// residual and the stop decision in Sw, pending until cg_reduce_dot_body
+// counts the iteration (res, prev, iter are read by the other blocks here and
+// may not change).  After a stop the partials are stale; then nothing is
+// recorded, and u is of no consequence.
 template <class VT, class AT>
 __device__ __forceinline__ void cg_u_body(const CgVecs<VT, AT>& v, int64_t n,
                                           const CgScalars* __restrict__ S, int64_t blk,
-                                          int64_t nblk) {
-    if (S->done) return;
+                                          int64_t nblk, const double* __restrict__ rpart = nullptr,
+                                          int nb = 0, CgScalars* Sw = nullptr) {
     using T = real_t<VT>;
-    const T beta = (T)((S->res * S->res) / (S->prev * S->prev));
+    double res, prev;
+    if (rpart) {
+        __shared__ double s_res;
+        if (threadIdx.x < 64) {
+            const double a = wave_sum_partials(rpart, nb, 1, 0);
+            if (threadIdx.x == 0) s_res = sqrt(a);
+        }
+        __syncthreads();
+        res = s_res;
+        prev = S->res;
+        const bool stop = S->iter + 1 >= S->maxiter || res <= S->tol;
+        if (blk == 0 && threadIdx.x == 0 && !Sw->done) {
+            Sw->res_new = res;
+            Sw->pending = 1;
+            if (stop) Sw->done = 1;
+        }
+        if (stop) return;
+    } else {
+        if (S->done) return;
+        res = S->res;
+        prev = S->prev;
+    }
+    const T beta = (T)((res * res) / (prev * prev));
     for (int64_t i = blk * blockDim.x + threadIdx.x; i < n; i += nblk * blockDim.x) {
         const VT a = v.r[i], w = v.u[i];
         VT nu;
@@ -176,8 +206,13 @@ template <class VT, class AT>
 __device__ __forceinline__ void cg_reduce_dot_body(const AT* __restrict__ partial, int G,
                                                    int64_t n, const CgVecs<VT, AT>& v,
                                                    double scale, double* __restrict__ part,
-                                                   const CgScalars* __restrict__ S, int blk,
-                                                   int nblk) {
+                                                   CgScalars* S, int blk, int nblk) {
+    if (blk == 0 && threadIdx.x == 0 && S->pending) {  // the iteration cg_u_body finished
+        S->prev = S->res;
+        S->res = S->res_new;
+        S->iter += 1;
+        S->pending = 0;
+    }
     if (S->done) return;
     using RA = real_t<AT>;
     __shared__ double s[RED_THREADS / 64];
@@ -317,21 +352,24 @@ void launch_cg_start(const float2* b, const float2* x_in, const CgVecs<VT, AT>& 
 }
 
 template <class VT, class AT>
-__global__ void cg_u_kernel(CgVecs<VT, AT> v, int64_t n, const CgScalars* __restrict__ S) {
-    cg_u_body(v, n, S, blockIdx.x, gridDim.x);
+__global__ void cg_u_kernel(CgVecs<VT, AT> v, int64_t n, const CgScalars* S, const double* __restrict__ rpart,
+                            int nb, CgScalars* Sw) {
+    cg_u_body(v, n, S, blockIdx.x, gridDim.x, rpart, nb, Sw);
 }
 
 template <class VT, class AT>
-void launch_cg_u(const CgVecs<VT, AT>& v, int64_t n, CgScalars* S, hipStream_t st) {
-    int grid = (int)std::min<int64_t>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL((cg_u_kernel<VT, AT>), dim3(grid), dim3(256), 0, st, v, n, S);
+void launch_cg_u(const CgVecs<VT, AT>& v, int64_t n, double* part, CgScalars* S, bool fold, hipStream_t st) {
+    // folding, every block reads the partials: at most two blocks per CU
+    const int grid = (int)std::min<int64_t>((n + 255) / 256, fold ? 512 : 4096);
+    hipLaunchKernelGGL((cg_u_kernel<VT, AT>), dim3(grid), dim3(256), 0, st, v, n, S,
+                       fold ? part + 2 * RED_BLOCKS : nullptr, red_grid(n), S);
     MSR_CHECK_LAUNCH();
 }
 
 template <class VT, class AT>
 __global__ void __launch_bounds__(RED_THREADS)
 cg_reduce_dot_kernel(const AT* __restrict__ partial, int G, int64_t n, CgVecs<VT, AT> v,
-                     double scale, double* __restrict__ part, const CgScalars* __restrict__ S) {
+                     double scale, double* __restrict__ part, CgScalars* S) {
     cg_reduce_dot_body(partial, G, n, v, scale, part, S, blockIdx.x, gridDim.x);
 }
 
@@ -371,13 +409,14 @@ cg_xr_step_kernel(CgVecs<VT, AT> v, int64_t n, const double* __restrict__ dpart,
 }
 
 template <class VT, class AT>
-void launch_cg_xr_step(const CgVecs<VT, AT>& v, int64_t n, double* part, CgScalars* S,
+void launch_cg_xr_step(const CgVecs<VT, AT>& v, int64_t n, double* part, CgScalars* S, bool finish,
                        hipStream_t st) {
     const int g = red_grid(n);
     double* rpart = part + 2 * RED_BLOCKS;
     hipLaunchKernelGGL((cg_xr_step_kernel<VT, AT>), dim3(g), dim3(RED_THREADS), 0, st, v, n, part,
                        g, rpart, S);
     MSR_CHECK_LAUNCH();
+    if (!finish) return;
     hipLaunchKernelGGL(cg_iter_finish, dim3(1), dim3(64), 0, st, rpart, g, S);
     MSR_CHECK_LAUNCH();
 }
@@ -437,17 +476,18 @@ void launch_cg_start_batch(const CgJob<VT, AT>* jobs, const int* pre, int nj, in
 
 template <class VT, class AT>
 __global__ void __launch_bounds__(RED_THREADS)
-cg_u_batch_kernel(const CgJob<VT, AT>* __restrict__ jobs, const int* __restrict__ pre, int nj) {
+cg_u_batch_kernel(const CgJob<VT, AT>* __restrict__ jobs, const int* __restrict__ pre, int nj, int fold) {
     const int j = batch_job(pre, nj, blockIdx.x);
     const CgJob<VT, AT>& J = jobs[j];
-    cg_u_body(J.v, J.n, J.S, (int64_t)blockIdx.x - pre[j], pre[j + 1] - pre[j]);
+    const int nb = pre[j + 1] - pre[j];
+    cg_u_body(J.v, J.n, J.S, (int64_t)blockIdx.x - pre[j], nb, fold ? J.part + 2 * RED_BLOCKS : nullptr, nb, J.S);
 }
 
 template <class VT, class AT>
-void launch_cg_u_batch(const CgJob<VT, AT>* jobs, const int* pre, int nj, int nblocks,
+void launch_cg_u_batch(const CgJob<VT, AT>* jobs, const int* pre, int nj, int nblocks, bool fold,
                        hipStream_t st) {
     hipLaunchKernelGGL((cg_u_batch_kernel<VT, AT>), dim3(nblocks), dim3(RED_THREADS), 0, st, jobs,
-                       pre, nj);
+                       pre, nj, (int)fold);
     MSR_CHECK_LAUNCH();
 }
 
@@ -462,18 +502,10 @@ cg_reduce_dot_batch_kernel(const CgJob<VT, AT>* __restrict__ jobs, const int* __
 }
 
 template <class VT, class AT>
-__global__ void cg_alpha_batch(const CgJob<VT, AT>* __restrict__ jobs, const int* __restrict__ pre) {
-    const int j = blockIdx.x;
-    cg_alpha_body(jobs[j].part, pre[j + 1] - pre[j], jobs[j].S);
-}
-
-template <class VT, class AT>
 void launch_cg_reduce_dot_batch(const CgJob<VT, AT>* jobs, const int* pre, int nj, int nblocks,
                                 hipStream_t st) {
     hipLaunchKernelGGL((cg_reduce_dot_batch_kernel<VT, AT>), dim3(nblocks), dim3(RED_THREADS), 0,
                        st, jobs, pre, nj);
-    MSR_CHECK_LAUNCH();
-    hipLaunchKernelGGL((cg_alpha_batch<VT, AT>), dim3(nj), dim3(64), 0, st, jobs, pre);
     MSR_CHECK_LAUNCH();
 }
 
@@ -482,22 +514,24 @@ __global__ void __launch_bounds__(RED_THREADS)
 cg_xr_batch_kernel(const CgJob<VT, AT>* __restrict__ jobs, const int* __restrict__ pre, int nj) {
     const int j = batch_job(pre, nj, blockIdx.x);
     const CgJob<VT, AT>& J = jobs[j];
-    cg_xr_body(J.v, J.n, J.part, J.S, blockIdx.x - pre[j], pre[j + 1] - pre[j]);
+    const int nb = pre[j + 1] - pre[j];
+    cg_xr_body(J.v, J.n, J.part + 2 * RED_BLOCKS, J.S, blockIdx.x - pre[j], nb, J.part, nb, J.S);
 }
 
 template <class VT, class AT>
 __global__ void cg_iter_finish_batch(const CgJob<VT, AT>* __restrict__ jobs,
                                      const int* __restrict__ pre) {
     const int j = blockIdx.x;
-    cg_iter_finish_body(jobs[j].part, pre[j + 1] - pre[j], jobs[j].S);
+    cg_iter_finish_body(jobs[j].part + 2 * RED_BLOCKS, pre[j + 1] - pre[j], jobs[j].S);
 }
 
 template <class VT, class AT>
-void launch_cg_xr_batch(const CgJob<VT, AT>* jobs, const int* pre, int nj, int nblocks,
+void launch_cg_xr_batch(const CgJob<VT, AT>* jobs, const int* pre, int nj, int nblocks, bool finish,
                         hipStream_t st) {
     hipLaunchKernelGGL((cg_xr_batch_kernel<VT, AT>), dim3(nblocks), dim3(RED_THREADS), 0, st, jobs,
                        pre, nj);
     MSR_CHECK_LAUNCH();
+    if (!finish) return;
     hipLaunchKernelGGL((cg_iter_finish_batch<VT, AT>), dim3(nj), dim3(64), 0, st, jobs, pre);
     MSR_CHECK_LAUNCH();
 }
@@ -523,20 +557,21 @@ void launch_to_f32_batch(const CgJob<double2, AT>* jobs, const int* pre, int nj,
     template void launch_cg_start<VT, AT>(const float2*, const float2*, const CgVecs<VT, AT>&,   \
                                           int64_t, bool, double*, CgScalars*, double, double,    \
                                           int, bool, hipStream_t);                               \
-    template void launch_cg_u<VT, AT>(const CgVecs<VT, AT>&, int64_t, CgScalars*, hipStream_t);  \
+    template void launch_cg_u<VT, AT>(const CgVecs<VT, AT>&, int64_t, double*, CgScalars*, bool, \
+                                      hipStream_t);                                              \
     template void launch_cg_reduce_dot<VT, AT>(const AT*, int, int64_t, const CgVecs<VT, AT>&,   \
                                                double, double*, CgScalars*, hipStream_t, bool);  \
     template void launch_cg_xr<VT, AT>(const CgVecs<VT, AT>&, int64_t, double*, CgScalars*,      \
                                        hipStream_t);                                             \
     template void launch_cg_xr_step<VT, AT>(const CgVecs<VT, AT>&, int64_t, double*, CgScalars*, \
-                                            hipStream_t);                                        \
+                                            bool, hipStream_t);                                  \
     template void launch_cg_start_batch<VT, AT>(const CgJob<VT, AT>*, const int*, int, int,      \
                                                 bool, bool, double, double, int, hipStream_t);   \
-    template void launch_cg_u_batch<VT, AT>(const CgJob<VT, AT>*, const int*, int, int,          \
+    template void launch_cg_u_batch<VT, AT>(const CgJob<VT, AT>*, const int*, int, int, bool,    \
                                             hipStream_t);                                        \
     template void launch_cg_reduce_dot_batch<VT, AT>(const CgJob<VT, AT>*, const int*, int, int, \
                                                      hipStream_t);                               \
-    template void launch_cg_xr_batch<VT, AT>(const CgJob<VT, AT>*, const int*, int, int,         \
+    template void launch_cg_xr_batch<VT, AT>(const CgJob<VT, AT>*, const int*, int, int, bool,   \
                                              hipStream_t);                                       \
     template void launch_epilogue_batch<VT, AT>(const CgJob<VT, AT>*, const int*, int, int,      \
                                                 hipStream_t);
