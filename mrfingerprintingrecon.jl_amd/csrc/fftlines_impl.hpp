@@ -2,8 +2,8 @@
 // per length by the fftlines_p*.hip translation units.
 #pragma once
 
-#include "fft.hpp"
 #include "fftlines.hpp"
+#include "wgfft.hpp"
 
 #include <cstdlib>
 
@@ -314,6 +314,138 @@ __global__ void __launch_bounds__(256) cols_kernel(LinePass p, const CT* __restr
     }
 }
 
+// ------------------------------------------------ lines by the workgroup
+// The same passes with the transform of wgfft.hpp: the first stage loads and the
+// last stage stores straight from global memory, two LDS round trips less, and
+// every thread holds 8 values or so where a wavefront plan with few threads per
+// line holds up to 40.  Bound: LDS traffic and barriers; stores of 8-byte values
+// go one by one.
+// Which is faster depends on the values per thread of the wavefront plan, v =
+// NF / T, and on the type.  On MI355X, per pass, wavefront -> workgroup:
+//  - ComplexF64, v > 8: rows 320 (v = 20) 681 -> 431 us, 384 (24) 1160 -> 523, 640 (40)
+//    122 -> 31, 120 (15) 49 -> 34, 300 (9) 17.1 -> 14.0, 600 (9) 34.5 -> 29.3; columns
+//    192 (24) 359 -> 196, 240 (15) 215 -> 136, 288 (9) 13.6 -> 12.3, but 576 (9)
+//    32.6 -> 38.4 and 600 (9) 35.3 -> 40.7: 4 columns a workgroup there.
+//  - ComplexF32, whose wavefront kernels move 16 bytes per access: rows 192 (24)
+//    30.5 -> 21.6, 96 (24) 15.0 -> 11.1, 120 (15) 19.5 -> 12.8, but at 160 to 600 points
+//    v up to 20 is faster by wavefronts (rows 400 70 -> 87, columns 200 14.9 -> 19.7,
+//    160 65 -> 76), and so is 72 (9: a 36 x 36 x 36 backprojection 311 -> 317).  From 960 points the wavefront kernels have few
+//    lines per workgroup (columns 1024 188 -> 141, rows 362 -> 290).
+//  - v = 8 (exact plans): columns 256 of the compact ComplexF64 3D apply 2.17 -> 2.64
+//    ms, ComplexF32 rows 512 75 -> 93 us: wavefronts.
+template <int N, class CT>
+constexpr bool lines_by_workgroup(bool rows) {
+    const int v = N / FFTPlan<N>::T;
+    if (sizeof(CT) == 16) return v > 8 && (rows || v > 10 || N <= 300);
+    return v > 20 || (v > 10 && (N <= 120 || N >= 960));
+}
+
+// input of bin q / output in bin q: the index placed there by select_bin, or
+// -1 (n of nf values placed by sel)
+__device__ __forceinline__ int placed_at(int q, int n, int nf, int sel) {
+    if (sel == SEL_FIRST) return q < n ? q : -1;
+    if (sel == SEL_CENTER) {
+        int i = q + n / 2;
+        if (i >= nf) i -= nf;
+        return i < n ? i : -1;
+    }
+    if (q < (n + 1) / 2) return q;
+    const int i = q - nf + n;
+    return i >= (n + 1) / 2 ? i : -1;
+}
+
+constexpr int wg_threads(int lines, int nf) { return ((lines * nf + WG_VALUES - 1) / WG_VALUES + 63) / 64 * 64; }
+
+template <int NF, class CT>
+constexpr int rows_wg_lines() {
+    const int want = (sizeof(CT) == 16 ? 2048 : 4096) / NF;
+    return want < 1 ? 1 : (want > 32 ? 32 : want);
+}
+
+template <int NF, int DIR, class CT>
+__global__ void __launch_bounds__((wg_threads(rows_wg_lines<NF, CT>(), NF)))
+rows_wg_kernel(LinePass p, const CT* __restrict__ tw) {
+    if (p.skip && *p.skip) return;
+    using RT = real_t<CT>;
+    constexpr int F = rows_wg_lines<NF, CT>();
+    __shared__ CT s[F * wg_pitch<NF, CT>()];
+    const int64_t l0 = (int64_t)blockIdx.x * F;
+    const int nl = (int)(p.nlines - l0 < F ? p.nlines - l0 : F);
+    const CT* in = static_cast<const CT*>(p.in) + l0 * p.in_pitch;
+    CT* out = static_cast<CT*>(p.out) + l0 * p.out_pitch;
+    wg_fft<NF, DIR, 0, 1, true, true, CT>(s, F, tw, false, false, 0,
+        [&](int l, int q) {
+            const int i = placed_at(q, p.lin, NF, p.isel);
+            if (i < 0 || l >= nl) return cz<CT>();
+            const CT v = in[l * p.in_pitch + i];
+            return p.win64 ? cscale(v, (RT)p.win64[i]) : p.win ? cscale(v, (RT)p.win[i]) : v;
+        },
+        [&](int, int, int l, int q, CT v) {
+            const int j = placed_at(q, p.lout, NF, p.sel);
+            if (j < 0 || l >= nl) return;
+            out[l * p.out_pitch + j] = p.w64 ? cscale(v, (RT)p.w64[j]) : p.w ? cscale(v, (RT)p.w[j]) : v;
+        });
+}
+
+// columns per workgroup: 64-byte pieces of a row or more, at most 1024 threads
+template <int NF, class CT>
+constexpr int cols_wg_shift() { return (NF <= 256 ? 3 : NF <= 1024 ? 2 : 1) + (sizeof(CT) == 16 ? 0 : 1); }
+
+template <int NF, int DIR, class CT>
+__global__ void __launch_bounds__((wg_threads(1 << cols_wg_shift<NF, CT>(), NF)))
+cols_wg_kernel(LinePass p, const CT* __restrict__ tw) {
+    if (p.skip && *p.skip) return;
+    using RT = real_t<CT>;
+    constexpr int SH = cols_wg_shift<NF, CT>(), WC = 1 << SH;
+    __shared__ CT s[WC * wg_pitch<NF, CT>()];
+    // neighbouring column tiles next to each other on one XCD (cols_kernel)
+    const unsigned nbx = gridDim.x, total = nbx * gridDim.y;
+    unsigned L = blockIdx.x + nbx * blockIdx.y;
+    if (L < total - total % 16u) L = (((L >> 4) << 3) + (L & 7u)) * 2u + ((L >> 3) & 1u);
+    const int64_t col0 = (int64_t)(L % nbx) * WC;
+    const int64_t b = L / nbx;
+    const int nc = (int)(p.ncols - col0 < WC ? p.ncols - col0 : WC);
+    const int64_t ibase = b * p.in_bstride + col0, obase = b * p.out_bstride + col0;
+    // the dense kernel store runs along the line, everything else across
+    wg_fft<NF, DIR, 0, 1, true, true, CT>(s, WC, tw, true, p.lam == nullptr, SH,
+        [&](int l, int q) {
+            const int i = placed_at(q, p.lin, NF, p.isel);
+            if (i < 0 || l >= nc) return cz<CT>();
+            const int64_t idx = ibase + i * p.in_stride + l;
+            CT v;
+            if constexpr (sizeof(CT) == 16)
+                v = p.in_compact ? st_load<CT, cx64>(static_cast<const cx64*>(p.in) + idx)
+                                 : static_cast<const CT*>(p.in)[idx];
+            else
+                v = static_cast<const CT*>(p.in)[idx];
+            return p.win64 ? cscale(v, (RT)p.win64[i]) : p.win ? cscale(v, (RT)p.win[i]) : v;
+        },
+        [&](int, int, int l, int q, CT v) {
+            const int j = placed_at(q, p.lout, NF, p.sel);
+            if (j < 0 || l >= nc) return;
+            if (p.w64) v = cscale(v, (RT)p.w64[j]);
+            else if (p.w) v = cscale(v, (RT)p.w[j]);
+            if (p.lam) {
+                // dense Toeplitz kernel, rounded once to ComplexF32 / Float32
+                const int64_t col = col0 + l;
+                const int64_t off = (col * p.P + b + p.p0) * p.lout + j;
+                const int64_t mi = p.lam3d ? (int64_t)j * p.ny2 * p.nx2 + col : (int64_t)j * p.nx2 + col;
+                const bool on = p.mask[mi] != 0;
+                if (p.lam_real) reinterpret_cast<float*>(p.lam)[off] = on ? (float)v.x : 0.f;
+                else reinterpret_cast<float2*>(p.lam)[off] = on ? make_float2((float)v.x, (float)v.y)
+                                                               : make_float2(0.f, 0.f);
+                return;
+            }
+            const int64_t idx = obase + j * p.out_stride + l;
+            if constexpr (sizeof(CT) == 16)
+                if (p.out_compact) {
+                    st_store<CT, cx64>(static_cast<cx64*>(p.out) + idx, v);
+                    return;
+                }
+            static_cast<CT*>(p.out)[idx] = v;
+        });
+}
+
 // MSR_COLS_SINGLE=1 in the environment: 8-byte line and column values one
 // per access (to compare with the paired accesses)
 inline bool cols_single_forced() {
@@ -323,24 +455,38 @@ inline bool cols_single_forced() {
 
 template <int N, class CT>
 void launch_rows_n(const LinePass& p, const CT* tw, hipStream_t st) {
-    constexpr int BLK = rows_block<N, CT>();
-    constexpr int F = BLK / FFTPlan<N>::T;
-    dim3 grid((unsigned)ceil_div(p.nlines, F));
-    LinePass q = p;
-    q.single = cols_single_forced() ? 1 : 0;
-    if (q.dir < 0) hipLaunchKernelGGL((rows_kernel<N, -1, CT>), grid, dim3(BLK), 0, st, q, tw);
-    else hipLaunchKernelGGL((rows_kernel<N, 1, CT>), grid, dim3(BLK), 0, st, q, tw);
+    if constexpr (lines_by_workgroup<N, CT>(true)) {
+        constexpr int F = rows_wg_lines<N, CT>();
+        const dim3 grid((unsigned)ceil_div(p.nlines, F)), blk(wg_threads(F, N));
+        if (p.dir < 0) hipLaunchKernelGGL((rows_wg_kernel<N, -1, CT>), grid, blk, 0, st, p, tw);
+        else hipLaunchKernelGGL((rows_wg_kernel<N, 1, CT>), grid, blk, 0, st, p, tw);
+    } else {
+        constexpr int BLK = rows_block<N, CT>();
+        constexpr int F = BLK / FFTPlan<N>::T;
+        dim3 grid((unsigned)ceil_div(p.nlines, F));
+        LinePass q = p;
+        q.single = cols_single_forced() ? 1 : 0;
+        if (q.dir < 0) hipLaunchKernelGGL((rows_kernel<N, -1, CT>), grid, dim3(BLK), 0, st, q, tw);
+        else hipLaunchKernelGGL((rows_kernel<N, 1, CT>), grid, dim3(BLK), 0, st, q, tw);
+    }
 }
 
 template <int N, class CT>
-void launch_cols_n(const LinePass& p0, const CT* tw, hipStream_t st) {
-    LinePass p = p0;
-    p.single = cols_single_forced() ? 1 : 0;
-    constexpr int WC = cols_wc<N, CT>();
-    constexpr int BLK = (WC * FFTPlan<N>::T) < 256 ? WC * FFTPlan<N>::T : 256;
-    dim3 grid((unsigned)ceil_div(p.ncols, WC), (unsigned)p.nb);
-    if (p.dir < 0) hipLaunchKernelGGL((cols_kernel<N, -1, CT>), grid, dim3(BLK), 0, st, p, tw);
-    else hipLaunchKernelGGL((cols_kernel<N, 1, CT>), grid, dim3(BLK), 0, st, p, tw);
+void launch_cols_n(const LinePass& p, const CT* tw, hipStream_t st) {
+    if constexpr (lines_by_workgroup<N, CT>(false)) {
+        constexpr int WC = 1 << cols_wg_shift<N, CT>();
+        const dim3 grid((unsigned)ceil_div(p.ncols, WC), (unsigned)p.nb), blk(wg_threads(WC, N));
+        if (p.dir < 0) hipLaunchKernelGGL((cols_wg_kernel<N, -1, CT>), grid, blk, 0, st, p, tw);
+        else hipLaunchKernelGGL((cols_wg_kernel<N, 1, CT>), grid, blk, 0, st, p, tw);
+    } else {
+        LinePass q = p;
+        q.single = cols_single_forced() ? 1 : 0;
+        constexpr int WC = cols_wc<N, CT>();
+        constexpr int BLK = (WC * FFTPlan<N>::T) < 256 ? WC * FFTPlan<N>::T : 256;
+        dim3 grid((unsigned)ceil_div(p.ncols, WC), (unsigned)p.nb);
+        if (q.dir < 0) hipLaunchKernelGGL((cols_kernel<N, -1, CT>), grid, dim3(BLK), 0, st, q, tw);
+        else hipLaunchKernelGGL((cols_kernel<N, 1, CT>), grid, dim3(BLK), 0, st, q, tw);
+    }
 }
 
 // Launch the rows (or cols) pass of p if its length is one of LIST: the body

@@ -6,8 +6,8 @@
 // the factors 3 and 5 leave no common power of two) holds up to 40 values per
 // thread.  The first stage can take its inputs from global memory and the last
 // one hand its outputs over in registers, a line's LDS round trip less at
-// either end.  Plans, twiddles and butterflies are those of fft.hpp, so both give
-// the same bits.
+// either end.  Plans, twiddles and butterflies are those of fft.hpp: the results
+// differ at most by the fused multiply-adds that the compiler chooses.
 #pragma once
 
 #include "fft.hpp"
