@@ -17,7 +17,8 @@
 // 9 (27) visits per sample) and the latency of the chain from sample to weight.
 // On MI355X, before (tiles of 32 x 32 or 16 x 8 x 8 cells in LDS, then a gather over
 // the padded tiles) and after: 256 x 256, K = 5 (15 pairs), 512 000 samples
-// 4.60 -> 0.66 ms; 80 x 72 x 64, K = 4 real, 320 000 samples 17.7 -> 6.8 ms.
+// 4.60 -> 0.60 ms; 80 x 72 x 64, K = 4 real, 320 000 samples 17.7 -> 5.1 ms, where taking
+// only the samples that reach the wave's plane gave 6.9 -> 5.1 (2D: 0.64 -> 0.60).
 #include "kernel_spread.hpp"
 
 #include <hipcub/hipcub.hpp>
@@ -111,7 +112,7 @@ kspread_gather_kernel(const int4* __restrict__ cells, const double* __restrict__
                       const int* __restrict__ first, const double* __restrict__ vals, int tiles, KernelGeom g,
                       int np, double2* __restrict__ grid) {
     constexpr int NR = D == 2 ? 6 : 18;  // runs of sorted samples, two per bin row
-    __shared__ int4 s_pt[4][64];         // {sample, packed offsets, frame, -} of a chunk
+    __shared__ int4 s_pt[4][72];         // {sample, offsets dx, dy dz, frame}: up to 7 left over and a chunk
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 15, q4 = lane >> 4, lx = r & 3, ly = r >> 2;
     // neighbouring tiles on one XCD
@@ -141,33 +142,43 @@ kspread_gather_kernel(const int4* __restrict__ cells, const double* __restrict__
     f64x4 acc[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
+    // samples left over from the chunk before, at the front of s_pt
+    int left = 0;
     for (int p0 = 0; p0 < total; p0 += 64) {
-        const int cnt = min(64, total - p0);
-        {
-            const int p = p0 + min(lane, cnt - 1);
-            int s = 0;
+        const int p = min(p0 + lane, total - 1);
+        int s = 0;
 #pragma unroll
-            for (int i = 0; i < NR; ++i)
-                if (p >= pre[i]) s = start[i] + p - pre[i];
-            const int4 c = cells[s];
-            // first cell of the tile relative to the sample's first, in -4 .. 7
-            int dx = X - c.x + 3, dy = Y - c.y + 3, dz = D == 3 ? Z - c.z + 3 : 0;
-            dx += dx < -4 ? g.n[0] : 0;
-            dx -= dx > 7 ? g.n[0] : 0;
-            dy += dy < -4 ? g.n[1] : 0;
-            dy -= dy > 7 ? g.n[1] : 0;
-            if (D == 3) {
-                dz += dz < -4 ? g.n[2] : 0;
-                dz -= dz > 7 ? g.n[2] : 0;
-            }
-            // a plane (3D) or slot out of reach takes no weight: offset 8
-            if (lane >= cnt || (D == 3 && (unsigned)dz > 7u)) dx = 8;
-            s_pt[wave][lane] = make_int4(s, dx, (dy & 0xFFFF) | (dz << 16), c.w);
+        for (int i = 0; i < NR; ++i)
+            if (p >= pre[i]) s = start[i] + p - pre[i];
+        const int4 c = cells[s];
+        // first cell of the tile relative to the sample's first, in -4 .. 7
+        int dx = X - c.x + 3, dy = Y - c.y + 3, dz = D == 3 ? Z - c.z + 3 : 0;
+        dx += dx < -4 ? g.n[0] : 0;
+        dx -= dx > 7 ? g.n[0] : 0;
+        dy += dy < -4 ? g.n[1] : 0;
+        dy -= dy > 7 ? g.n[1] : 0;
+        if (D == 3) {
+            dz += dz < -4 ? g.n[2] : 0;
+            dz -= dz > 7 ? g.n[2] : 0;
+        }
+        // keep the samples whose support meets the tile, 121 of 144 cells of
+        // the bins around (3D: the plane, 968 of 1728), in their order
+        const bool reach = p0 + lane < total && dx > -4 && dy > -4 && (D == 2 || (unsigned)dz <= 7u);
+        const uint64_t kept = __ballot(reach);
+        const int at = left + __builtin_amdgcn_mbcnt_hi((unsigned)(kept >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((unsigned)kept, 0u));
+        if (reach) s_pt[wave][at] = make_int4(s, dx, (dy & 0xFFFF) | (dz << 16), c.w);
+        left += __popcll(kept);
+        int use = left & ~7;
+        if (p0 + 64 >= total) {  // the last chunk: fill up with samples of no weight (offset 8)
+            use = (left + 7) & ~7;
+            if (lane < use - left) s_pt[wave][left + lane] = make_int4(s, 8, 0, c.w);
+            left = use;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (int q = 0; q < cnt; q += 8) {
+        for (int q = 0; q < use; q += 8) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int4 e = s_pt[wave][q + 4 * h + q4];
@@ -182,8 +193,13 @@ kspread_gather_kernel(const int4* __restrict__ cells, const double* __restrict__
                     acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[m * 16], b, acc[m], 0, 0, 0);
             }
         }
+        left -= use;
+        int4 e = make_int4(0, 8, 0, 0);
+        if (lane < left) e = s_pt[wave][use + lane];
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (lane < left) s_pt[wave][lane] = e;
     }
     const int64_t G = (int64_t)g.n[0] * g.n[1] * (D == 3 ? g.n[2] : 1);
     double2* dst = grid + ((int64_t)Z * g.n[1] + Y + ly) * g.n[0] + X + lx;
