@@ -92,3 +92,17 @@ def test_constructions_on_threads_and_streams(torch, msr):
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_pairs_in_several_chunks(torch, msr):
+    """64 x 64 x 64, K = 6: the FP64 grids of 21 pairs exceed the construction's
+    budget, so the pairs go in chunks of whole row tiles; every pair has the
+    bits of a construction that takes it in one chunk."""
+    N = (64, 64, 64)
+    trj, U = protocol(N, 6, 3, 400, False)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    build = lambda u: msr.NFFTNormalOp(N, dev(trj), dev(u)).prod.A.Λ
+    lam = build(U)
+    pairs = [d for d in range(lam.ndim) if lam.shape[d] == 21][0]
+    assert torch.equal(lam.narrow(pairs, 0, 15), build(U[:5]))
+    assert torch.equal(lam.narrow(pairs, 20, 1).flatten(), build(U[5:]).flatten())
