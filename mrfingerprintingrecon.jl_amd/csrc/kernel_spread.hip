@@ -17,8 +17,9 @@
 // 9 (27) visits per sample) and the latency of the chain from sample to weight.
 // On MI355X, before (tiles of 32 x 32 or 16 x 8 x 8 cells in LDS, then a gather over
 // the padded tiles) and after: 256 x 256, K = 5 (15 pairs), 512 000 samples
-// 4.60 -> 0.60 ms; 80 x 72 x 64, K = 4 real, 320 000 samples 17.7 -> 5.1 ms, where taking
-// only the samples that reach the wave's plane gave 6.9 -> 5.1 (2D: 0.64 -> 0.60).
+// 4.60 -> 0.60 ms; 80 x 72 x 64, K = 4 real, 320 000 samples 17.7 -> 3.0 ms (all 10
+// pairs in one row tile); taking only the samples that reach the wave's plane gave 2.54
+// ms per launch after 3.47 (2D: 0.60 after 0.64).
 #include "kernel_spread.hpp"
 
 #include <hipcub/hipcub.hpp>
