@@ -18,6 +18,7 @@
 #include "fft.hpp"
 #include "fftlines.hpp"
 #include "planes.hpp"
+#include "search.hpp"
 #include "spread.hpp"
 
 namespace msr {
@@ -187,13 +188,7 @@ __global__ void fwd_region_kernel(const float* __restrict__ kc, int64_t M, FwdGe
 
 // first position of a sorted key >= v
 __device__ __forceinline__ int lower_bound(const int* __restrict__ sorted, int n, int v) {
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (sorted[mid] < v) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
+    return lower_bound_at(n, v, [&](int i) { return sorted[i]; });
 }
 
 // first[r] = first sample of region r (r <= nr), nb[r] = its batches

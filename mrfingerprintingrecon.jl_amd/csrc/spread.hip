@@ -15,6 +15,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include "search.hpp"
 #include "spread.hpp"
 
 namespace msr {
@@ -83,13 +84,7 @@ __global__ void bin_id_kernel(const float* __restrict__ kc, int d, int64_t M, Pl
 __global__ void sorted_first_kernel(const int* __restrict__ sorted, int n, int nkeys, int* __restrict__ first) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b > nkeys) return;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (sorted[mid] < b) lo = mid + 1;
-        else hi = mid;
-    }
-    first[b] = lo;
+    first[b] = lower_bound_at(n, b, [&](int i) { return sorted[i]; });
 }
 
 void sorted_first(const int* sorted, int64_t n, int64_t nkeys, int* first, hipStream_t st) {
