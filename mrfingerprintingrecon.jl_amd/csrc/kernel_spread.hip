@@ -22,6 +22,8 @@
 // ms per launch after 3.47 (2D: 0.60 after 0.64).
 #include "kernel_spread.hpp"
 
+#include "blockgrid.hpp"
+
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -106,7 +108,7 @@ __global__ void kspread_values_kernel(ValueSrc src, int np, int tiles, double* _
     }
 }
 
-// blockIdx.y: group of MT row tiles
+// blockIdx.z: group of MT row tiles; blocks are counted over x and y (split_blocks)
 template <int D, int MT, bool REAL>
 __global__ void __launch_bounds__(256)
 kspread_gather_kernel(const int4* __restrict__ cells, const double* __restrict__ wts,
@@ -117,11 +119,11 @@ kspread_gather_kernel(const int4* __restrict__ cells, const double* __restrict__
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 15, q4 = lane >> 4, lx = r & 3, ly = r >> 2;
     // neighbouring tiles on one XCD
-    const int64_t nblk = gridDim.x;
-    int64_t lb = nblk % 8 ? (int64_t)blockIdx.x : (int64_t)(blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8;
+    const int64_t nblk = (int64_t)gridDim.x * gridDim.y, b = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    int64_t lb = nblk % 8 ? b : (b % 8) * (nblk / 8) + b / 8;
     if (D == 2) lb = lb * 4 + wave;
     const int nbx = g.nb[0], nby = g.nb[1], nbz = D == 3 ? g.nb[2] : 1;
-    if (lb >= (int64_t)nbx * nby * nbz) return;  // (2D: a wave without a tile; waves never synchronise)
+    if (lb >= (int64_t)nbx * nby * nbz) return;  // (a wave without a tile; waves never synchronise)
     const int tx = (int)(lb % nbx), ty = (int)(lb / nbx % nby), tz = (int)(lb / ((int64_t)nbx * nby));
     const int X = 4 * tx, Y = 4 * ty, Z = D == 3 ? 4 * tz + wave : 0;
     // the runs: bins tx - 1 .. tx + 1 of each bin row, cut where x wraps
@@ -139,7 +141,7 @@ kspread_gather_kernel(const int4* __restrict__ cells, const double* __restrict__
         pre[2 * i + 1] = total;
         if (b1 >= b0) total += first[row + b1 + 1] - start[2 * i + 1];
     }
-    const int mt0 = blockIdx.y * MT;
+    const int mt0 = blockIdx.z * MT;
     f64x4 acc[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
@@ -294,7 +296,8 @@ void KernelSpread::run(const ValueSrc& src, int np, double2* grid, hipStream_t s
     hipLaunchKernelGGL(kspread_values_kernel, dim3(gv), dim3(256), 0, st, src, np, tiles, vals.as<double>());
     MSR_CHECK_LAUNCH();
     const int64_t nblk = d == 2 ? ceil_div((int64_t)nb[0] * nb[1], 4) : (int64_t)nb[0] * nb[1] * nb[2];
-    const dim3 gr((unsigned)nblk, (unsigned)groups);
+    const BlockGrid xy = split_blocks(nblk, 256);
+    const dim3 gr(xy.x, xy.y, (unsigned)groups);
 #define MSR_KGATHER(DD, MM, RR)                                                                           \
     hipLaunchKernelGGL((kspread_gather_kernel<DD, MM, RR>), gr, dim3(256), 0, st, cells.as<int4>(),       \
                        wts.as<double>(), first.as<int>(), vals.as<double>(), tiles, g, np, grid)

@@ -106,3 +106,22 @@ def test_pairs_in_several_chunks(torch, msr):
     pairs = [d for d in range(lam.ndim) if lam.shape[d] == 21][0]
     assert torch.equal(lam.narrow(pairs, 0, 15), build(U[:5]))
     assert torch.equal(lam.narrow(pairs, 20, 1).flatten(), build(U[5:]).flatten())
+
+
+def test_grid_of_more_blocks_than_one_dimension_takes(torch, msr, monkeypatch):
+    """256 x 256 x 256: the 1024-point spreading grid has 2^24 output tiles of 256
+    threads, one more than a launch takes in one dimension.  Against the tile
+    spreading of the same samples (both FP64, rounded to Float32: 1e-7)."""
+    N = (256, 256, 256)
+    trj, U = protocol(N, 1, 2, 1000, True)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    A = msr.NFFTNormalOp(N, dev(trj), dev(U))
+    lam, km = A.prod.A.Λ, A.prod.A.kmask_indcs
+    del A
+    monkeypatch.setenv("MSR_SPREAD3D_SLAB_BUDGET", "1")
+    B = msr.NFFTNormalOp(N, dev(trj), dev(U))
+    assert torch.equal(km, B.prod.A.kmask_indcs)
+    ref = B.prod.A.Λ.double()
+    e = float((lam.double() - ref).norm() / ref.norm())
+    print(f"kernel {N}: gather against tiles {e:.2e}", flush=True)
+    assert e < 1e-7
