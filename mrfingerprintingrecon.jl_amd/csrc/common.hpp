@@ -30,13 +30,17 @@ struct Error : std::runtime_error {
     throw Error(code, buf);
 }
 
+// A failed call is reported here and once: hipGetLastError keeps returning it,
+// whatever succeeds after it, so the next launch check would report it again.
 #define MSR_HIP(call)                                                                    \
     do {                                                                                 \
         hipError_t e_ = (call);                                                          \
-        if (e_ != hipSuccess)                                                            \
+        if (e_ != hipSuccess) {                                                          \
+            (void)hipGetLastError();                                                     \
             ::msr::fail(e_ == hipErrorOutOfMemory ? MSR_ERR_NOMEM : MSR_ERR_HIP,         \
                         "%s failed: %s (%s:%d)", #call, hipGetErrorString(e_), __FILE__, \
                         __LINE__);                                                       \
+        }                                                                                \
     } while (0)
 
 #define MSR_CHECK_LAUNCH() MSR_HIP(hipGetLastError())

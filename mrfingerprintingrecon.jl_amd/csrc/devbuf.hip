@@ -7,6 +7,7 @@
 // before its release, as hipFree would have waited, so any stream or thread
 // may take it; at most IDLE_LIMIT bytes stay idle per device, oldest freed
 // first, and all of them when an allocation fails or a context is destroyed.
+#include <cstdlib>
 #include <mutex>
 #include <vector>
 
@@ -46,12 +47,21 @@ struct OnDevice {
         if (before >= 0) (void)hipSetDevice(before);
     }
 };
+
+// MSR_DEVICE_ALLOC_LIMIT=<bytes> in the environment: larger requests fail, as on
+// a device without that much free memory (a check of the paths taken then)
+bool over_limit(size_t n) {
+    const char* e = getenv("MSR_DEVICE_ALLOC_LIMIT");
+    return e && n > (size_t)strtoull(e, nullptr, 10);
+}
 }  // namespace
 
 void* dev_acquire(size_t n, size_t& cap, int& device) {
     MSR_HIP(hipGetDevice(&device));
     cap = (n + 511) / 512 * 512;
-    {
+    if (over_limit(cap)) {
+        cap = SIZE_MAX / 4;  // more than any device has: fails below
+    } else {
         Idle& c = idle();
         std::lock_guard<std::mutex> guard(c.mu);
         size_t best = c.blocks.size();

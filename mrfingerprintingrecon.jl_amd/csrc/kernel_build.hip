@@ -253,8 +253,8 @@ void op_build_from_traj(msr_normalop* op, const msr_traj* traj, const void* U, i
     const int pc4 = chunk((size_t)4 << 30);
     try {
         grids();
-    } catch (const Error&) {
-        if (pc4 == pc) throw;
+    } catch (const Error& e) {
+        if (e.code != MSR_ERR_NOMEM || pc4 == pc) throw;
         pc = pc4;
         A.release();
         grids();

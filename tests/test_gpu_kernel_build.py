@@ -125,3 +125,22 @@ def test_grid_of_more_blocks_than_one_dimension_takes(torch, msr, monkeypatch):
     e = float((lam.double() - ref).norm() / ref.norm())
     print(f"kernel {N}: gather against tiles {e:.2e}", flush=True)
     assert e < 1e-7
+
+
+def test_less_memory_than_the_larger_budget(torch, msr, monkeypatch):
+    """64 x 64 x 64, K = 6 with requests above 3 GiB failing: the 4 GiB grids of 16
+    pairs cannot be had, so the pairs go in chunks of 8, with the same bits; the
+    failed allocation does not show up in a later call either.  With nothing
+    large enough the construction fails as out of memory, and the next works."""
+    N = (64, 64, 64)
+    trj, U = protocol(N, 6, 3, 400, False)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    build = lambda: msr.NFFTNormalOp(N, dev(trj), dev(U)).prod.A.Λ
+    lam = build()
+    monkeypatch.setenv("MSR_DEVICE_ALLOC_LIMIT", str(3 << 30))
+    assert torch.equal(lam, build())
+    monkeypatch.setenv("MSR_DEVICE_ALLOC_LIMIT", str(64 << 20))
+    with pytest.raises(Exception, match="out of memory"):
+        build()
+    monkeypatch.delenv("MSR_DEVICE_ALLOC_LIMIT")
+    assert torch.equal(lam, build())
