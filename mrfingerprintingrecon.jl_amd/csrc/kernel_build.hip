@@ -225,9 +225,10 @@ void op_build_from_traj(msr_normalop* op, const msr_traj* traj, const void* U, i
     const bool f64 = true;
     const size_t es = f64 ? sizeof(double2) : sizeof(float2);
     // output-owned gather on the matrix cores; the tile spreading takes grids
-    // of less than three bins (and, for comparison, builds under
-    // MSR_SPREAD3D_SLAB_BUDGET)
-    const bool gather = kernel_spread_supported(d, n4) && !getenv("MSR_SPREAD3D_SLAB_BUDGET");
+    // of less than three bins (and, for comparison, all grids under
+    // MSR_KERNEL_TILES=1)
+    const char* tiled = getenv("MSR_KERNEL_TILES");
+    const bool gather = kernel_spread_supported(d, n4) && !(tiled && atoi(tiled));
     KernelSpread ks;
     const SpreadPlan* plan = nullptr;
     if (gather) ks.build(traj, n4, st);

@@ -156,7 +156,9 @@ def test_3d_spreading_atomic_and_slab_paths_agree(torch, msr, monkeypatch):
     """3D tile spreading stores padded tiles to a slab summed by a gather, or,
     when one channel group's slab exceeds the budget (forced here with
     MSR_SPREAD3D_SLAB_BUDGET=1), adds them into the grid with atomics: kernel
-    and backprojection agree between the two paths and with the oracle."""
+    (under MSR_KERNEL_TILES=1, which sends the construction to the tiles) and
+    backprojection agree between the two paths and with the oracle, the kernel
+    also with the construction's own gather, whatever the budget."""
     N = (16, 16, 16)
     trj, U, cm, x = kooshball_case(N, 2, 3, 6, 5)
     cml = [dev(torch, c) for c in cm]
@@ -168,15 +170,20 @@ def test_3d_spreading_atomic_and_slab_paths_agree(torch, msr, monkeypatch):
         b = msr.calculate_backprojection(dev(torch, data), dev(torch, trj), cml, U=dev(torch, U))
         return A.prod.A.Λ.cpu().numpy(), b.cpu().numpy()
 
+    lam_g, _ = run()
+    monkeypatch.setenv("MSR_KERNEL_TILES", "1")
     lam_s, b_s = run()
     monkeypatch.setenv("MSR_SPREAD3D_SLAB_BUDGET", "1")
     lam_a, b_a = run()
+    monkeypatch.delenv("MSR_KERNEL_TILES")
+    assert np.array_equal(run()[0], lam_g)  # the budget is the tiles' alone
     monkeypatch.delenv("MSR_SPREAD3D_SLAB_BUDGET")
     lam_ref, _ = toeplitz.toeplitz_kernel(N, trj, U)
     b_ref = toeplitz.backprojection(data, trj, cm, U=U)
     print(f"3d paths: kernel slab/atomic {rel_err(lam_s, lam_a):.1e}, bp {rel_err(b_s, b_a):.1e}; "
           f"vs oracle {rel_err(lam_a, lam_ref):.1e} {rel_err(b_a, b_ref):.1e}", flush=True)
     assert rel_err(lam_s, lam_a) < 1e-7 and rel_err(b_s, b_a) < 1e-6
+    assert rel_err(lam_g, lam_s) < 1e-7
     assert rel_err(lam_a, lam_ref) < 3e-7 and rel_err(b_a, b_ref) < 2e-6
 
 

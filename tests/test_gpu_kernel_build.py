@@ -118,6 +118,7 @@ def test_grid_of_more_blocks_than_one_dimension_takes(torch, msr, monkeypatch):
     A = msr.NFFTNormalOp(N, dev(trj), dev(U))
     lam, km = A.prod.A.Λ, A.prod.A.kmask_indcs
     del A
+    monkeypatch.setenv("MSR_KERNEL_TILES", "1")
     monkeypatch.setenv("MSR_SPREAD3D_SLAB_BUDGET", "1")
     B = msr.NFFTNormalOp(N, dev(trj), dev(U))
     assert torch.equal(km, B.prod.A.kmask_indcs)
