@@ -228,37 +228,43 @@ void op_build_from_traj(msr_normalop* op, const msr_traj* traj, const void* U, i
     // of less than three bins (and, for comparison, all grids under
     // MSR_KERNEL_TILES=1)
     const char* tiled = getenv("MSR_KERNEL_TILES");
-    const bool gather = kernel_spread_supported(d, n4) && !(tiled && atoi(tiled));
+    bool gather = kernel_spread_supported(d, n4) && !(tiled && atoi(tiled));
     KernelSpread ks;
     const SpreadPlan* plan = nullptr;
-    if (gather) ks.build(traj, n4, st);
-    else plan = &spread_plan(traj, n4, st);
-    auto slab = [&](int nch) { return gather ? 0 : spread_workspace_bytes(*plan, nch, f64); };
-    const size_t per_ch = es * (size_t)G4 + std::max(es * (size_t)(G4 / 2), slab(1));
-    // pairs per chunk: as many as the budget holds, less what would begin a
+    // Pairs per chunk: as many as the budget holds, less what would begin a
     // row tile of the gather, whose cost is by the tile (16 real or 8 complex
     // pairs).  6 GiB stay idle between constructions; where that much is not
     // there, 4 GiB.  At 80 x 72 x 64, K = 4 real (10 pairs, 5.7 GB) 6 GiB take one
     // chunk, 4 GiB took chunks of 7 and 3 (gather 5.1 -> 3.0 ms, construction 9.5 -> 7.4).
-    const int tile = gather ? (u_real ? 16 : 8) : 1;
-    auto chunk = [&](size_t budget) {
-        const int c = (int)std::max<size_t>(1, std::min<size_t>((size_t)P, budget / per_ch));
-        return c < P && c > tile ? c - c % tile : c;
-    };
-    int pc = chunk((size_t)(gather ? 6 : 4) << 30);
+    // The gather's tables come on top, 64 d + 16 bytes per sample; where they do
+    // not fit, the tiles do without.
+    int pc = 0;
     DevBuf A, B;
-    auto grids = [&] {
+    auto slab = [&](int nch) { return gather ? 0 : spread_workspace_bytes(*plan, nch, f64); };
+    auto prepare = [&](size_t budget) {
+        if (gather) ks.build(traj, n4, st);
+        else plan = &spread_plan(traj, n4, st);
+        const size_t per_ch = es * (size_t)G4 + std::max(es * (size_t)(G4 / 2), slab(1));
+        const int tile = gather ? (u_real ? 16 : 8) : 1;
+        const int c = (int)std::max<size_t>(1, std::min<size_t>((size_t)P, budget / per_ch));
+        pc = c < P && c > tile ? c - c % tile : c;
         A.alloc(es * (size_t)pc * G4);
         B.alloc(std::max(es * (size_t)pc * (G4 / 2), slab(pc)));
+        if (gather) ks.reserve(src, pc);
     };
-    const int pc4 = chunk((size_t)4 << 30);
-    try {
-        grids();
-    } catch (const Error& e) {
-        if (e.code != MSR_ERR_NOMEM || pc4 == pc) throw;
-        pc = pc4;
-        A.release();
-        grids();
+    for (int gib = gather ? 6 : 4;; gib = 4) {
+        try {
+            prepare((size_t)gib << 30);
+            break;
+        } catch (const Error& e) {
+            if (e.code != MSR_ERR_NOMEM || !gather) throw;
+            A.release();
+            B.release();
+            if (gib == 4) {
+                gather = false;
+                ks.release();
+            }
+        }
     }
 
     const size_t ls = op->lam_real ? sizeof(float) : sizeof(float2);

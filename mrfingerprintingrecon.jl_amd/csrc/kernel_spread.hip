@@ -240,6 +240,7 @@ static KernelGeom geom_of(const KernelSpread& k) {
 }
 
 void KernelSpread::build(const msr_traj* traj, const int64_t* grid_n, hipStream_t st) {
+    if (built) return;
     d = traj->d;
     M = traj->M;
     MSR_REQUIRE(M < (int64_t)INT32_MAX, MSR_ERR_UNSUPPORTED, "more than 2^31 samples");
@@ -281,17 +282,36 @@ void KernelSpread::build(const msr_traj* traj, const int64_t* grid_n, hipStream_
                            traj->frame.as<int>(), perm.as<int>(), M, g, cells.as<int4>(), wts.as<double>());
     MSR_CHECK_LAUNCH();
     MSR_HIP(hipStreamSynchronize(st));  // temporaries are freed on return
+    built = true;
+}
+
+void KernelSpread::release() {
+    for (DevBuf* b : {&cells, &wts, &first, &vals}) b->release();
+    built = false;
+}
+
+// Row tiles of np channels: MT per wave, in groups.
+struct KernelTiles {
+    int mt, groups;
+};
+static KernelTiles tiles_of(const ValueSrc& src, int np) {
+    const int tiles = (int)ceil_div(np, src.u_real ? 16 : 8);
+    const int mt = tiles == 1 ? 1 : (tiles == 2 ? 2 : 4);
+    return {mt, (int)ceil_div(tiles, mt)};
+}
+
+void KernelSpread::reserve(const ValueSrc& src, int np) {
+    const KernelTiles t = tiles_of(src, np);
+    const size_t vb = sizeof(double) * 16 * (size_t)src.nt * t.groups * t.mt;
+    if (vals.bytes < vb) vals.alloc(vb);
 }
 
 void KernelSpread::run(const ValueSrc& src, int np, double2* grid, hipStream_t st) {
     MSR_REQUIRE(src.kind == 1 && src.U, MSR_ERR_ERROR, "the kernel's spreading takes basis pair products");
     const KernelGeom g = geom_of(*this);
-    int tiles = (int)ceil_div(np, src.u_real ? 16 : 8);
-    const int mt = tiles == 1 ? 1 : (tiles == 2 ? 2 : 4);
-    const int groups = (int)ceil_div(tiles, mt);
-    tiles = groups * mt;
-    const size_t vb = sizeof(double) * 16 * (size_t)src.nt * tiles;
-    if (vals.bytes < vb) vals.alloc(vb);
+    const auto [mt, groups] = tiles_of(src, np);
+    const int tiles = groups * mt;
+    reserve(src, np);
     const int gv = (int)std::min<int64_t>((src.nt * tiles * 16 + 255) / 256, 4096);
     hipLaunchKernelGGL(kspread_values_kernel, dim3(gv), dim3(256), 0, st, src, np, tiles, vals.as<double>());
     MSR_CHECK_LAUNCH();

@@ -17,7 +17,12 @@ struct KernelSpread {
     DevBuf wts;     // (M, d, 8) double: ES weights of the cells c - 3 .. c + 4
     DevBuf first;   // (bins + 1) int32: first sorted sample of a bin
     DevBuf vals;    // pair products per frame (basis values only)
+    bool built = false;
+    // Once; again does nothing, unless an allocation failed.
     void build(const msr_traj* traj, const int64_t* grid, hipStream_t st);
+    void release();  // the tables
+    // Room for the values of up to np channels of src.
+    void reserve(const ValueSrc& src, int np);
     // grid (np, prod n) ComplexF64, overwritten: channel p = sum over samples of
     // conj(U[t, pair_j]) U[t, pair_k] times the weights (src.kind 1); real
     // values for a real basis

@@ -145,3 +145,23 @@ def test_less_memory_than_the_larger_budget(torch, msr, monkeypatch):
         build()
     monkeypatch.delenv("MSR_DEVICE_ALLOC_LIMIT")
     assert torch.equal(lam, build())
+
+
+def test_less_memory_than_the_samples_tables(torch, msr, monkeypatch):
+    """200 000 samples on a 16 x 15 image with requests above 8 MB failing: the
+    gather's 25.6 MB of weights cannot be had, the tile spreading takes the
+    construction (both FP64, rounded to ComplexF32: 1e-7)."""
+    N = (16, 15)
+    trj, U = protocol(N, 3, 4, 50000, False)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    trj, U = dev(trj), dev(U)
+    build = lambda: msr.NFFTNormalOp(N, trj, U).prod.A
+    A = build()
+    monkeypatch.setenv("MSR_KERNEL_TILES", "1")
+    T = build()
+    monkeypatch.delenv("MSR_KERNEL_TILES")
+    monkeypatch.setenv("MSR_DEVICE_ALLOC_LIMIT", str(8 << 20))
+    B = build()
+    assert torch.equal(A.kmask_indcs, B.kmask_indcs)
+    assert torch.equal(B.Λ, T.Λ)
+    assert rel_err(A.Λ.cpu().numpy(), B.Λ.cpu().numpy()) < 1e-7
