@@ -89,6 +89,15 @@ int msr_version(void);
 int msr_ctx_create(int device, msr_ctx **out);
 int msr_ctx_destroy(msr_ctx *ctx);
 
+/* Gives the device memory back that the library keeps for its next buffers:
+ * freed temporaries and buffers of destroyed handles, up to 8 GiB per device
+ * (blocks of 512 MiB or more only while an eighth of its memory is free).
+ * The library does so by itself when an allocation of its own fails and when a
+ * context is destroyed; a program whose other allocations run short calls this.
+ * *freed (may be NULL): the bytes given back.  Memory of live handles stays.
+ * No reference counterpart: CUDA.jl's CUDA.reclaim(). */
+int msr_trim(msr_ctx *ctx, size_t *freed);
+
 /* --------------------------------------------------------- trajectories */
 /* Sample selection shared by the kernel build and the backprojection:
  * trj[:, sample_mask] and the per-frame sample counts / offsets

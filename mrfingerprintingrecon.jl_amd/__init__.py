@@ -32,7 +32,7 @@ __all__ = ["NFFTNormalOp", "calculate_backprojection", "forward", "cg", "cg_", "
            "kernel_key", "save_kernel", "load_kernel", "kernel_file_info", "KernelCache",
            "reconstruct_coilwise", "calibration_region", "calibration_kspace",
            "calculate_coil_maps", "default_calib_size", "FFTNormalOp", "save_tuning",
-           "load_tuning"]
+           "load_tuning", "trim"]
 
 _ctxs = {}
 
@@ -528,6 +528,14 @@ def load_tuning(path, device=None):
     entries; ArgumentError for a file measured on another device type."""
     n = ctypes.c_int()
     _lib.call("msr_tune_load", _ctx(_dev_index(device)), os.fsencode(path), ctypes.byref(n))
+    return n.value
+
+
+def trim(device=None):
+    """Gives the device memory back that the library keeps for its next buffers
+    (msr_trim), for the program's other allocations.  Returns the bytes."""
+    n = ctypes.c_size_t()
+    _lib.call("msr_trim", _ctx(_dev_index(device)), ctypes.byref(n))
     return n.value
 
 

@@ -57,6 +57,7 @@ SIGNATURES = {
     "msr_version": (_I, []),
     "msr_ctx_create": (_I, [_I, _P]),
     "msr_ctx_destroy": (_I, [_P]),
+    "msr_trim": (_I, [_P, _P]),
     "msr_traj_create": (_I, [_P, _I, _I64, _I64, _P, _P, _P, _P]),
     "msr_traj_info": (_I, [_P, _P, _P]),
     "msr_traj_destroy": (_I, [_P]),

@@ -137,6 +137,15 @@ int msr_ctx_destroy(msr_ctx* ctx) {
     });
 }
 
+int msr_trim(msr_ctx* ctx, size_t* freed) {
+    return guarded([&] {
+        MSR_NOTNULL(ctx);
+        ensure_device(ctx);
+        const size_t bytes = dev_trim(ctx->device);
+        if (freed) *freed = bytes;
+    });
+}
+
 int msr_traj_create(msr_ctx* ctx, int d, int64_t nsamp, int64_t nt, const float* trj,
                     const uint8_t* mask, void* stream, msr_traj** out) {
     return guarded([&] {

@@ -40,8 +40,8 @@ namespace msr {
 void* dev_acquire(size_t n, size_t& cap, int& device);
 // Waits for the device (as hipFree does), then keeps or frees the block.
 void dev_release(void* p, size_t cap, int device) noexcept;
-// Frees the idle blocks of the device.
-void dev_trim(int device) noexcept;
+// Frees the idle blocks of the device; their bytes.
+size_t dev_trim(int device) noexcept;
 
 // Device buffer with RAII free.
 struct DevBuf {

@@ -1,0 +1,76 @@
+"""Device memory kept for the library's next buffers: bounded, given back on
+request, and nothing large kept while the device is nearly full."""
+import gc
+
+import numpy as np
+import pytest
+
+from conftest import load_package
+
+pytestmark = pytest.mark.gpu
+
+N, K = (64, 64, 64), 3          # a construction's FP64 grids: 1.6 and 0.8 GB
+GRIDS = 6 * 256 ** 3 * 16 * 3 // 2
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return torch
+
+
+@pytest.fixture(scope="module")
+def msr():
+    return load_package()
+
+
+def kernel(torch, msr):
+    rng = np.random.default_rng(0)
+    trj = torch.from_numpy(rng.uniform(-0.5, 0.5, size=(4, 200, 3)).astype(np.float32)).cuda()
+    U = torch.from_numpy(rng.normal(size=(K, 4)).astype(np.float32)).cuda()
+    lam = msr.NFFTNormalOp(N, trj, U).prod.A.Λ
+    gc.collect()
+    torch.cuda.synchronize()
+    return lam
+
+
+def available(torch):
+    torch.cuda.empty_cache()
+    return torch.cuda.mem_get_info()[0]
+
+
+def test_trim_gives_idle_memory_back(torch, msr):
+    first = kernel(torch, msr)       # tables and contexts that stay
+    msr.trim()
+    before = available(torch)
+    again = kernel(torch, msr)
+    assert torch.equal(first, again)
+    del again
+    kept = before - available(torch)
+    freed = msr.trim()
+    after = available(torch)
+    print(f"kept {kept >> 20} MiB, freed {freed >> 20} MiB, {before - after >> 20} MiB remain", flush=True)
+    assert freed >= GRIDS and kept >= GRIDS
+    assert before - after < 32 << 20
+    assert msr.trim() == 0
+    assert torch.equal(first, kernel(torch, msr))
+
+
+def test_nothing_large_stays_while_the_device_is_nearly_full(torch, msr):
+    first = kernel(torch, msr)
+    msr.trim()
+    free, total = torch.cuda.mem_get_info()
+    rest = total // 16
+    if free < rest:
+        pytest.skip("device in use")
+    hold = torch.empty(free - rest, dtype=torch.uint8, device="cuda")
+    try:
+        assert torch.equal(first, kernel(torch, msr))
+        freed = msr.trim()
+    finally:
+        del hold
+        torch.cuda.empty_cache()
+    print(f"freed {freed >> 20} MiB", flush=True)
+    assert freed < GRIDS // 4
