@@ -74,3 +74,25 @@ def test_nothing_large_stays_while_the_device_is_nearly_full(torch, msr):
         torch.cuda.empty_cache()
     print(f"freed {freed >> 20} MiB", flush=True)
     assert freed < GRIDS // 4
+
+
+def test_an_operator_takes_what_its_footprint_says(torch, msr):
+    """The construction leaves idle blocks a fifth larger than the operator's
+    intermediates (120 MiB, 100 MiB needed): its buffers take blocks of their own
+    size, at most 1/64 and 64 KiB more than its footprint counts."""
+    n, k = (256, 256), 5
+    trj = torch.from_numpy(msr.synth.traj_2d_radial_goldenratio(512, 8, 40)).cuda()
+    U = torch.from_numpy(msr.synth.t2_basis(40, k)).cuda()
+    maps = [torch.randn(n[::-1], dtype=torch.complex64, device="cuda") for _ in range(20)]
+    msr.trim()
+    A = msr.NFFTNormalOp(n, trj, U, cmaps=maps)
+    gc.collect()
+    own, kernel_bytes = msr.footprint(A, "f32")
+    msr.trim()
+    with_op = available(torch)
+    del A
+    gc.collect()
+    msr.trim()
+    used = available(torch) - with_op
+    print(f"used {used / 2**20:.1f} MiB, footprint {(own + kernel_bytes) / 2**20:.1f} MiB", flush=True)
+    assert used <= (own + kernel_bytes) * 65 / 64 + (1 << 20)
