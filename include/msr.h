@@ -197,7 +197,7 @@ int msr_backprojection_channelwise(msr_ctx *ctx, const msr_traj *traj, int d,
  * x: (N..., K) ComplexF32 device; U: (Nt, K) or NULL for I(Nt); cmaps: ncoils
  * device pointers or NULL (one coil, S = 1).  out: (nsamp, nt, C) ComplexF32;
  * samples removed by the trajectory's mask are written as 0.  Synchronises
- * the stream (its workspace, kept on the trajectory, is free on return). */
+ * the stream (its workspace is released on return). */
 int msr_forward(msr_ctx *ctx, const msr_traj *traj, int d, const int64_t *img_shape,
                 const void *x, int K, const void *U, int u_real, int ncoils,
                 const void *const *cmaps, void *out, void *stream);

@@ -213,8 +213,9 @@ __global__ void fwd_batch_kernel(const int* __restrict__ first, const int* __res
 }
 
 // Samples sorted by region (stable) and cut into batches, once per trajectory
-// and grid.
+// and grid; only the building holds the handle.
 static const FwdPlan& fwd_plan(const msr_traj* traj, const FwdGeom& g, hipStream_t st) {
+    std::lock_guard<std::recursive_mutex> lock(traj->mu);
     std::array<int64_t, 2> key{g.n[0], g.n[1]};
     auto it = traj->fwd_plans.find(key);
     if (it != traj->fwd_plans.end()) return *it->second;
@@ -375,10 +376,6 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
         Gos *= nos[a];
     }
     const int nch = C * K;
-    // the plan and the workspace belong to the handle: hold it until the call's
-    // kernels have run (allocated and freed on every call, the workspace took up to
-    // 12 ms of a call with 3.9 ms of kernels)
-    std::lock_guard<std::recursive_mutex> lock(traj->mu);
     const FwdGeom g{{nos[0], nos[1], nos[2]}};
     const FwdPlan* plan = nullptr;
     if (d == 2 && U && nos[0] <= 1024 && nos[1] <= 1024 && traj->M > 0) {
@@ -389,13 +386,15 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
     const bool maps = ncoils >= 1 && cmaps;
     const size_t mb = maps ? (sizeof(float2) * (size_t)C * V + 255) / 256 * 256 : 0;
     // workspace: coil maps, then S_c x_k and two grid buffers, or (matrix
-    // cores) the row transforms and the grid in groups of 8 coils
+    // cores) the row transforms and the grid in groups of 8 coils.  The call's
+    // own, from the idle blocks: calls on one trajectory run side by side, and
+    // nothing stays with the handle (128 x 128 x 128, 16 coils, K = 4: 18 GB)
     const size_t zb = plan ? 0 : sizeof(float2) * (size_t)nch * V;
     const size_t ab = plan ? (sizeof(float2) * (size_t)nch * nos[0] * NN[1] + 255) / 256 * 256
                            : sizeof(float2) * (size_t)nch * Gos;
     const size_t bb = plan ? sizeof(float2) * (size_t)K * CB * PLANE_COIL_GROUP * Gos : ab;
-    DevBuf& work = traj->fwd_work;
-    if (work.bytes < mb + zb + ab + bb) work.alloc(mb + zb + ab + bb);
+    DevBuf work;
+    work.alloc(mb + zb + ab + bb);
     float2* mp = maps ? work.as<float2>() : nullptr;
     float2* Z = reinterpret_cast<float2*>(work.as<char>() + mb);
     float2* A = reinterpret_cast<float2*>(work.as<char>() + mb + zb);
@@ -440,7 +439,7 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
                            plan->batches.as<int4>(), plan->nbatch, plan->nry, nsel,
                            reinterpret_cast<const float*>(B), g, K, C, U, u_real, traj->nt, (float2*)out);
         MSR_CHECK_LAUNCH();
-        MSR_HIP(hipStreamSynchronize(st));  // the workspace is free again
+        MSR_HIP(hipStreamSynchronize(st));  // the workspace is freed on return
         return;
     }
     int grid = (int)std::min<int64_t>(((int64_t)nch * V + 255) / 256, 16384);
@@ -512,7 +511,7 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
                            traj->frame.as<int>(), traj->sel.p ? traj->sel.as<int64_t>() : nullptr,
                            traj->M, nsel, Gfin, g, K, C, U, u_real, traj->nt, (float2*)out);
     MSR_CHECK_LAUNCH();
-    MSR_HIP(hipStreamSynchronize(st));  // the workspace is free again
+    MSR_HIP(hipStreamSynchronize(st));  // the workspace is freed on return
 }
 
 }  // namespace msr

@@ -144,7 +144,6 @@ struct msr_traj {
     std::vector<int64_t> nsamp_t;     // host copy of the per-frame counts
     mutable std::map<std::array<int64_t, 3>, std::unique_ptr<msr::SpreadPlan>> plans;
     mutable msr::DevBuf bp_work;      // backprojection workspace (grow-only)
-    mutable msr::DevBuf fwd_work;     // forward-model workspace (grow-only)
     mutable std::map<std::array<int64_t, 2>, std::unique_ptr<msr::FwdPlan>> fwd_plans;
     bool integer = false;             // created from integer (Cartesian) k-space indices
     mutable std::map<std::array<int64_t, 3>, std::unique_ptr<msr::CartPlan>> cart_plans;

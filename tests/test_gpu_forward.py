@@ -5,6 +5,9 @@ batch and batches that do not fill, coil counts around the groups of 8, real
 and complex bases, masked samples, and the shapes that keep one wavefront per
 sample (few coils, sparse samples, U = I).  Tolerance 1e-5 relative L2 (W = 8
 spreading in ComplexF32), as the other NUFFT tests."""
+import gc
+import threading
+
 import numpy as np
 import pytest
 
@@ -60,3 +63,64 @@ def test_forward_matches_oracle(torch, msr, N, K, C, nt, ns, real, masked):
     msr.forward(dev(x), traj, cmaps=[dev(cm[0])], U=dev(U))
     again = msr.forward(dev(x), traj, cmaps=[dev(c) for c in cm], U=dev(U))
     assert torch.equal(first, again)
+
+
+def problem(torch, N, K, C, nt, ns, seed=5):
+    """x, trajectory, maps and U on the device."""
+    rng = np.random.default_rng(seed)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    c = lambda *sh: (rng.normal(size=sh) + 1j * rng.normal(size=sh)).astype(np.complex64)
+    trj = rng.uniform(-0.5, 0.5, size=(nt, ns, len(N))).astype(np.float32)
+    return dev(c(K, *N[::-1])), dev(trj), [dev(m) for m in c(C, *N[::-1])], dev(c(K, nt))
+
+
+@pytest.mark.parametrize("N,K,C", [((256, 256), 4, 16), ((64, 64, 64), 2, 8)])
+def test_workspace_goes_back(torch, msr, N, K, C):
+    """2D (matrix cores) and 3D: after a call, nothing of its workspace (at least
+    the grids' 134 and 268 MB) stays with the trajectory."""
+    x, trj, cm, U = problem(torch, N, K, C, 8, 3000)
+    traj = msr.plan_trajectory(trj)
+    msr.forward(x, traj, cmaps=cm[:4], U=U)   # tables and the plan
+    torch.cuda.synchronize()
+
+    def available():
+        gc.collect()
+        torch.cuda.empty_cache()
+        msr.trim()
+        return torch.cuda.mem_get_info()[0]
+
+    before = available()
+    msr.forward(x, traj, cmaps=cm, U=U)
+    left = before - available()
+    print(f"{left >> 20} MiB stay", flush=True)
+    assert left < 32 << 20
+
+
+def test_calls_on_one_trajectory_side_by_side(torch, msr):
+    """Threads with streams of their own, 2D and 3D handles shared: the bits of
+    the calls one after another."""
+    jobs = []
+    for N, K, C in [((48, 40), 3, 9), ((24, 20, 16), 2, 5)]:
+        x, trj, cm, U = problem(torch, N, K, C, 6, 500)
+        traj = msr.plan_trajectory(trj)
+        jobs += [(x, traj, cm[:c], U) for c in (C, 4)]
+    want = [msr.forward(x, t, cmaps=cm, U=U) for x, t, cm, U in jobs]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        st = torch.cuda.Stream()
+        x, t, cm, U = jobs[i]
+        with torch.cuda.stream(st):
+            for _ in range(10):
+                y = msr.forward(x, t, cmaps=cm, U=U)
+                st.synchronize()
+                if not torch.equal(y, want[i]):
+                    wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
