@@ -219,7 +219,6 @@ static const FwdPlan& fwd_plan(const msr_traj* traj, const FwdGeom& g, hipStream
     std::array<int64_t, 2> key{g.n[0], g.n[1]};
     auto it = traj->fwd_plans.find(key);
     if (it != traj->fwd_plans.end()) return *it->second;
-    MSR_REQUIRE(traj->M < (int64_t)INT32_MAX, MSR_ERR_UNSUPPORTED, "more than 2^31 samples");
     auto p = std::make_unique<FwdPlan>();
     const int M = (int)traj->M;
     p->nry = (int)ceil_div(g.n[1], FW_TY);
@@ -336,13 +335,20 @@ interp_mfma_kernel(const float* __restrict__ kc, const int* __restrict__ frame, 
     }
 }
 
-// Whether the batches pay: a batch costs the same however many samples it
+// Whether the batches can pay, which decides if they are made at all: from 4
+// coils on (the grid is stored for whole groups of 8), for grids that the fused
+// placement takes, and for sample counts whose batches, 64 threads each, stay
+// below the 2^32 threads of a launch.
+static bool fwd_batches_possible(const msr_traj* traj, const int64_t* nos, int C) {
+    return C >= 4 && nos[0] <= 1024 && nos[1] <= 1024 && traj->M > 0 && traj->M <= (int64_t)1 << 29;
+}
+
+// Whether they do pay: a batch costs the same however many samples it
 // holds, 0.43 ns per coefficient and 8 coils at full rate against 0.27 ns per
 // sample, coefficient and 4 coils of the one-wavefront-per-sample kernel
-// (measured 3.43 ms at 512 000 samples, 20 coils, K = 5).  From 4 coils on: the
-// grid is stored for whole groups of 8.
+// (measured 3.43 ms at 512 000 samples, 20 coils, K = 5).
 static bool fwd_batches_pay(int64_t nbatch, int64_t M, int C) {
-    return C >= 4 && 8 * nbatch * ceil_div(C, 8) <= 5 * M * ceil_div(C, 4);
+    return 8 * nbatch * ceil_div(C, 8) <= 5 * M * ceil_div(C, 4);
 }
 
 // Device copy of the coil maps, packed (C, V): one launch per 32 coils.
@@ -378,7 +384,7 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
     const int nch = C * K;
     const FwdGeom g{{nos[0], nos[1], nos[2]}};
     const FwdPlan* plan = nullptr;
-    if (d == 2 && U && nos[0] <= 1024 && nos[1] <= 1024 && traj->M > 0) {
+    if (d == 2 && U && fwd_batches_possible(traj, nos, C)) {
         plan = &fwd_plan(traj, g, st);
         if (!fwd_batches_pay(plan->nbatch, traj->M, C)) plan = nullptr;
     }

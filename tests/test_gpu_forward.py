@@ -96,6 +96,25 @@ def test_workspace_goes_back(torch, msr, N, K, C):
     assert left < 32 << 20
 
 
+def test_few_coils_make_no_plan(torch, msr):
+    """Three coils never take the matrix cores: 4 million samples are not sorted for
+    them, and no sorted list (16 MB, and the batches) stays with the trajectory."""
+    x, trj, cm, U = problem(torch, (32, 32), 1, 3, 4, 1000000)
+    traj = msr.plan_trajectory(trj)
+    msr.forward(x, msr.plan_trajectory(trj[:, :10].contiguous()), cmaps=cm, U=U)   # tables
+
+    def available():
+        gc.collect()
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        msr.trim()
+        return torch.cuda.mem_get_info()[0]
+
+    before = available()
+    msr.forward(x, traj, cmaps=cm, U=U)
+    assert before - available() < 8 << 20
+
+
 def test_calls_on_one_trajectory_side_by_side(torch, msr):
     """Threads with streams of their own, 2D and 3D handles shared: the bits of
     the calls one after another."""
