@@ -157,20 +157,28 @@ interp_kernel(const float* __restrict__ kc, const int* __restrict__ frame,
 // as 33 v_mfma_f32_16x16x4f32, four neighbouring cells along qy per step: lane
 // (r = lane mod 16, s = lane div 16) supplies float r of cell s (the grid is
 // stored [k][coil group][qx][qy][8 coils], so a step's 64 lanes read 256
-// consecutive bytes) and the weight w_x w_y of cell s for sample r.  Each
-// accumulator holds two coils of one sample and is folded with U[t_j, k] before
-// the next coefficient.  A step's grid values are loaded one (coil group,
-// coefficient) ahead.
+// consecutive bytes) and the weight w_x w_y of cell s for sample r.  The rows
+// of cells go to four accumulators in turn, each of which holds two coils of one
+// sample, the middle columns (the largest weights) last; their sum is folded
+// with U[t_j, k], in Float64, before the next coefficient.  A step's grid values
+// are loaded one (coil group, coefficient) ahead.
+//
+// Error: one accumulator for all 132 products and a fold in Float32 gave 1.03 to
+// 1.08 times the error against 64 bits of the lane tree below (interp_kernel);
+// this form 0.997 to 1.002 times (32 x 32 to 500 x 500, K = 1 to 8).
 //
 // Bound: matrix-core issue (33 x 32 cycles per 16 samples, coefficient and 8
 // coils; the 64 cells of a kernel are 48 % of the region's 132, and a region
 // away from the centre fills about 12 of the 16 columns).  At 256 x 256, 20
 // coils, K = 5, 512 000 samples on MI355X: interpolation
-// 3.43 -> 0.55 ms, a call with its FFTs 4.11 -> 0.68 ms
+// 3.43 -> 0.55 ms, a call with its FFTs 4.11 -> 0.68 ms.  Three waves per SIMD:
+// with four the accumulators lie in AGPRs and the call takes 0.72 ms (320 x 240, 32
+// coils, 2.02 ms for 1.88; 384 x 384, 16 coils, the other way, 0.54 for 0.55).
 constexpr int FW_TX = 4, FW_TY = 5;                      // region (floor cells)
 constexpr int FW_RX = FW_TX + 7, FW_RY = (FW_TY + 7) / 4;  // rows, column quads it reaches
 constexpr int FW_STEPS = FW_RX * FW_RY;
 static_assert(FW_RY * 4 == FW_TY + 7, "the columns of a region come in quads");
+constexpr int FW_ACC = 4;                                // accumulators
 constexpr int FW_PTS = 16;                               // samples per batch
 
 __global__ void fwd_region_kernel(const float* __restrict__ kc, int64_t M, FwdGeom g, int nry,
@@ -262,7 +270,7 @@ static const FwdPlan& fwd_plan(const msr_traj* traj, const FwdGeom& g, hipStream
 
 using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
 
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 interp_mfma_kernel(const float* __restrict__ kc, const int* __restrict__ frame, const int64_t* __restrict__ sel,
                    const int* __restrict__ perm, const int4* __restrict__ batches, int nbatch, int nry,
                    int64_t nsel, const float* __restrict__ G, FwdGeom g, int K, int C,
@@ -307,27 +315,33 @@ interp_mfma_kernel(const float* __restrict__ kc, const int* __restrict__ frame, 
     const float* b0 = base(0);
 #pragma unroll
     for (int st = 0; st < FW_STEPS; ++st) a[st] = load(b0, st);
-    float2 y[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+    double2 y[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
     int k = 0, cb = 0;
     for (int q = 0; q < ng; ++q) {
         const float* nb = base(q + 1 < ng ? q + 1 : q);
         float2 u;
         if (u_real) u = make_float2(reinterpret_cast<const float*>(U)[t + (int64_t)k * nt], 0.f);
         else u = reinterpret_cast<const float2*>(U)[t + (int64_t)k * nt];
-        f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        f32x4 z[FW_ACC];
 #pragma unroll
-        for (int st = 0; st < FW_STEPS; ++st) {
-            z = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st], wx[st / FW_RY] * wy[st % FW_RY], z, 0, 0, 0);
+        for (int i = 0; i < FW_ACC; ++i) z[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int o = 0; o < FW_STEPS; ++o) {
+            constexpr int quad[FW_RY] = {0, 2, 1};  // the middle columns, the largest weights, last
+            const int st = o % FW_RX * FW_RY + quad[o / FW_RX];
+            f32x4& zi = z[st / FW_RY % FW_ACC];
+            zi = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st], wx[st / FW_RY] * wy[st % FW_RY], zi, 0, 0, 0);
             a[st] = load(nb, st);
         }
-        cfma(y[0], u, make_float2(z[0], z[1]));
-        cfma(y[1], u, make_float2(z[2], z[3]));
+        const f32x4 zs = (z[0] + z[1]) + (z[2] + z[3]);
+        cfma(y[0], cto<double2>(u), make_double2(zs[0], zs[1]));
+        cfma(y[1], cto<double2>(u), make_double2(zs[2], zs[3]));
         if (++k == K) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int c = cb * PLANE_COIL_GROUP + 2 * s + h;
-                if (on && c < C) out[idx + (int64_t)c * nsel] = y[h];
-                y[h] = make_float2(0.f, 0.f);
+                if (on && c < C) out[idx + (int64_t)c * nsel] = cto<float2>(y[h]);
+                y[h] = make_double2(0.0, 0.0);
             }
             k = 0;
             ++cb;
