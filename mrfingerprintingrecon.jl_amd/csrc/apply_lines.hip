@@ -20,6 +20,7 @@
 // fused passes.  The arithmetic and the grids are ComplexF32 or ComplexF64
 // (the compact 8-byte storage of the fused 2D passes maps to ComplexF64 here).
 #include <algorithm>
+#include <cstdlib>
 
 #include "fftlines.hpp"
 #include "normalop.hpp"
@@ -135,7 +136,10 @@ static unsigned lines_grid(int64_t n) {
 
 int lines_chunk_coils(const msr_normalop* op) {
     // the two grids of a chunk in ComplexF64 stay within 2 x 1 GiB (at least
-    // one coil per chunk)
+    // one coil per chunk); MSR_COIL_CHUNK=<coils> lowers it (a check of the sums
+    // over chunks at small sizes)
+    const char* e = getenv("MSR_COIL_CHUNK");
+    if (e && atoi(e) >= 1) return std::min(atoi(e), op->C);
     int64_t g = op->K;
     for (int a = 0; a < op->d; ++a) g *= 2 * op->N[a];
     const int64_t per = g * (int64_t)sizeof(double2);

@@ -70,6 +70,29 @@ def test_toeplitz_matches_oracle(torch, msr, monkeypatch, N, K, C, real, identit
     assert rel_err(y.cpu().numpy().reshape(x.shape), ref) < 2e-6
 
 
+@pytest.mark.parametrize("path", ["MSR_APPLY_PLANES", "MSR_APPLY_LINES"])
+@pytest.mark.parametrize("N,K,C,chunk,identity", [
+    ((64, 48), 5, 7, 3, False),          # chunks of 3, 3 and 1 coils, summed in 3 groups
+    ((45, 27), 2, 5, 4, False),
+    ((20, 18, 15), 3, 5, 2, False),
+    ((12, 10, 9), 2, 4, 1, False),       # one coil at a time
+    ((24, 20), 3, 1, 1, True),
+])
+def test_coils_in_chunks(torch, msr, monkeypatch, path, N, K, C, chunk, identity):
+    """The coils of an operator too large for one pass, taken a chunk at a time."""
+    lam, km, cm, x = make_case(np.random.default_rng(6), N, K, C, identity=identity)
+    monkeypatch.setenv(path, "1")
+    monkeypatch.setenv("MSR_COIL_CHUNK", str(chunk))
+    A = msr.NFFTNormalOp(N, dev(torch, lam), dev(torch, km + 1),
+                         cmaps=None if cm is None else [dev(torch, c) for c in cm])
+    ref = toeplitz.apply_normal(N, lam.astype(np.complex128), km, None if cm is None else cm.astype(np.complex128),
+                                x.astype(np.complex128))
+    check(torch, A, x, ref)
+    y = torch.empty(x.size, dtype=torch.complex64, device="cuda")
+    A.A.mul_(y, dev(torch, x).reshape(-1), percoil=True)
+    assert rel_err(y.cpu().numpy().reshape(x.shape), ref) < 2e-6
+
+
 @pytest.mark.parametrize("N,K,C,real", [
     ((5, 4), 2, 3, False),               # one stage each
     ((3, 25), 1, 1, True),
