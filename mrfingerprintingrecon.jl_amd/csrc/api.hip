@@ -95,6 +95,13 @@ static int guarded(F&& f) {
     }
 }
 
+// Any stream may have used a handle's buffers: destroying it waits for the device.
+template <class Handle>
+static void destroy(Handle* h) {
+    DoneScope done(dev_wait());
+    delete h;
+}
+
 #define MSR_NOTNULL(p) MSR_REQUIRE((p) != nullptr, MSR_ERR_ARGUMENT, "%s is NULL", #p)
 
 extern "C" {
@@ -168,7 +175,7 @@ int msr_traj_destroy(msr_traj* traj) {
     return guarded([&] {
         if (!traj) return;
         ensure_device(traj->ctx);
-        delete traj;
+        destroy(traj);
     });
 }
 
@@ -274,7 +281,7 @@ int msr_normalop_destroy(msr_normalop* op) {
     return guarded([&] {
         if (!op) return;
         ensure_device(op->ctx);
-        delete op;
+        destroy(op);
     });
 }
 
@@ -424,7 +431,7 @@ int msr_batch_destroy(msr_batch* batch) {
     return guarded([&] {
         if (!batch) return;
         ensure_device(batch->ctx);
-        delete batch;
+        destroy(batch);
     });
 }
 
@@ -527,7 +534,7 @@ int msr_server_destroy(msr_server* server) {
     return guarded([&] {
         if (!server) return;
         ensure_device(server->ctx);
-        delete server;
+        destroy(server);
     });
 }
 
@@ -620,7 +627,10 @@ int msr_kernel_cache_create(msr_ctx* ctx, size_t budget_bytes, const char* direc
 
 int msr_kernel_cache_destroy(msr_kernel_cache* cache) {
     return guarded([&] {
-        if (cache) kernel_cache_destroy(cache);
+        if (!cache) return;
+        ensure_device(cache_ctx(cache));
+        DoneScope done(dev_wait());
+        kernel_cache_destroy(cache);
     });
 }
 

@@ -54,7 +54,7 @@ msr_traj* cart_traj_create(msr_ctx* ctx, int d, int64_t nsamp, int64_t nt, const
     MSR_REQUIRE(nsamp >= 1 && nt >= 1, MSR_ERR_ARGUMENT, "empty trajectory (%lld x %lld)",
                 (long long)nsamp, (long long)nt);
     const int64_t n = (int64_t)d * nsamp * nt;
-    DevBuf tf, bad;
+    TempBuf tf{st}, bad{st};
     tf.alloc(sizeof(float) * n);
     bad.alloc(sizeof(int));
     fill_floats(bad.p, 1, 0.f, st);
@@ -116,7 +116,7 @@ const CartPlan& cart_plan(const msr_traj* traj, const int64_t* N, int d, hipStre
     MSR_REQUIRE(traj->M < (int64_t)INT32_MAX && p->G < (int64_t)INT32_MAX, MSR_ERR_UNSUPPORTED,
                 "more than 2^31 samples or cells");
     const int M = (int)traj->M;
-    DevBuf cell, cell_s, idx, counts, temp;
+    TempBuf cell{st}, cell_s{st}, idx{st}, counts{st}, temp{st};
     cell.alloc(sizeof(int) * M);
     cell_s.alloc(sizeof(int) * M);
     idx.alloc(sizeof(int) * M);
@@ -293,7 +293,7 @@ __global__ void kmask_scatter_kernel(const uint8_t* __restrict__ flag, const int
 
 // kmask (1-based, ascending) from the per-cell flags
 static void cart_kmask(msr_normalop* op, const uint8_t* flag, int64_t G, hipStream_t st) {
-    DevBuf c, pos, temp;
+    TempBuf c{st}, pos{st}, temp{st};
     c.alloc(sizeof(int) * (G + 1));
     pos.alloc(sizeof(int) * (G + 1));
     MSR_HIP(hipMemsetAsync(c.p, 0, c.bytes, st));
@@ -326,7 +326,7 @@ void cart_build_kernel(msr_normalop* op, const msr_traj* traj, const uint8_t* M,
     CartN g{{op->N[0], op->N[1], op->N[2]}};
     const size_t es = u_real ? sizeof(float) : sizeof(float2);
     op->lam->alloc(es * (size_t)K * K * G);
-    DevBuf flag;
+    TempBuf flag{st};
     flag.alloc(G);
     const int grid = (int)std::min<int64_t>((G + 255) / 256, 16384);
     if (traj) {
@@ -370,7 +370,7 @@ void cart_load_dense(msr_normalop* op, const void* lambda, hipStream_t st) {
     const int KK = op->K * op->K;
     const size_t es = op->lam_real ? sizeof(float) : sizeof(float2);
     op->lam->alloc(es * (size_t)KK * G);
-    DevBuf flag;
+    TempBuf flag{st};
     flag.alloc(G);
     const int grid = (int)std::min<int64_t>((G * KK + 255) / 256, 16384);
     if (op->lam_real)
@@ -660,7 +660,7 @@ void cart_backprojection(msr_ctx* ctx, const msr_traj* traj, int d, const int64_
     }
     const CartPlan& plan = cart_plan(traj, N, d, st);
     const int64_t nch = (int64_t)ncoils * K;
-    DevBuf work;
+    TempBuf work{st};
     work.alloc(2 * sizeof(float2) * (size_t)nch * V);
     float2* Gd = work.as<float2>();
     float2* H = Gd + nch * V;
@@ -673,7 +673,7 @@ void cart_backprojection(msr_ctx* ctx, const msr_traj* traj, int d, const int64_
     // inverse FFT with fftshifted output: Gd -> H (3D through Gd)
     cart_fft(ctx, d, N, nch, Gd, H, Gd, +1, SEL_CENTER, false, nullptr, st);
     // the host staging array lives until the stream synchronisation below
-    DevBuf ptrs;
+    TempBuf ptrs{st};
     std::vector<const float2*> hp;
     if (cmaps) {
         hp.resize(ncoils);

@@ -101,7 +101,7 @@ void calib_kspace(msr_ctx* ctx, int d, const int64_t* Nc, int ncoils, const floa
                     "calibration k-space needs an FFT of length %lld", (long long)n[a]);
     }
     const int64_t V = n[0] * n[1] * n[2], total = V * ncoils;
-    DevBuf tmp;
+    TempBuf tmp{st};
     tmp.alloc(sizeof(float2) * (size_t)total);
     float2* T = tmp.as<float2>();
     const int grid = (int)std::min<int64_t>((total + 255) / 256, 4096);
@@ -160,7 +160,7 @@ void reconstruct_coilwise(msr_ctx* ctx, const msr_traj* traj, int d, const int64
     MSR_REQUIRE(ncoils >= 1, MSR_ERR_ARGUMENT, "ncoils = %d", ncoils);
     MSR_REQUIRE(niter >= 0, MSR_ERR_ARGUMENT, "Niter_cg = %d", niter);
     MSR_REQUIRE(prec_valid(prec), MSR_ERR_ARGUMENT, "precision = %d", prec);
-    DevBuf ones;
+    TempBuf ones{st};
     if (U == nullptr) {
         ones.alloc(sizeof(float) * (size_t)traj->nt);
         fill_floats(ones.p, traj->nt, 1.f, st);
@@ -172,7 +172,7 @@ void reconstruct_coilwise(msr_ctx* ctx, const msr_traj* traj, int d, const int64
     op_build_from_traj(op.get(), traj, U, u_real, st);
     op_alloc_scratch(op.get());
     const int64_t V = op->V;
-    DevBuf xbp;
+    TempBuf xbp{st};
     xbp.alloc(sizeof(float2) * (size_t)ncoils * V);
     backprojection(ctx, traj, d, N, data, ncoils, 1, U, u_real, nullptr, MSR_DCF_NONE, nullptr,
                    xbp.p, st, false);
@@ -192,7 +192,11 @@ void reconstruct_coilwise(msr_ctx* ctx, const msr_traj* traj, int d, const int64
         bs[c] = xbp.as<float2>() + (size_t)c * V;
     }
     batch_cg(bt.get(), xs.data(), bs.data(), niter, 0.0, 0.0, true, MSR_CG_DEVICE, prec, st);
-    MSR_HIP(hipStreamSynchronize(st));  // the workspaces are released on return
+    MSR_HIP(hipStreamSynchronize(st));
+    DoneScope done(true);  // the operators worked on this stream alone
+    bt.reset();
+    more.clear();
+    op.reset();
 }
 
 }  // namespace msr

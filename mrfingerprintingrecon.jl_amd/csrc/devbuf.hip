@@ -3,11 +3,13 @@
 // 0.6 GB at 256 x 256, K = 5) spent as long in them as in its kernels, and
 // with other allocations on the device up to 10 times that (measured 7 to
 // 24 ms per construction for 5 ms of kernels in 2D, 28 to 520 ms for 22 ms in
-// 3D).  A block is kept only after the device has finished everything queued
-// before its release, as hipFree would have waited, so any stream or thread
-// may take it; at most IDLE_LIMIT bytes stay idle per device, oldest freed
-// first, and no large block while the device is nearly full.  All are given back when an allocation of this library fails, when a context is
-// destroyed, and by msr_trim (another allocator in the process cannot ask).
+// 3D).  A released block is handed out again once nothing queued before its
+// release can use it: a temporary's at once (its function has waited for its
+// stream), a destroyed handle's too (destroying waits for the device), any other
+// after such a wait.  At most IDLE_LIMIT bytes are kept per device, oldest freed
+// first, and no large block while the device is nearly full.  All are given back
+// when an allocation of this library fails, when a context is destroyed, and by
+// msr_trim (another allocator in the process cannot ask).
 #include <cstdlib>
 #include <mutex>
 #include <vector>
@@ -41,6 +43,7 @@ struct Block {
     void* p;
     size_t cap;
     int device;
+    bool done;  // nothing queued uses it
 };
 struct Idle {
     std::mutex mu;
@@ -74,6 +77,53 @@ bool over_limit(size_t n) {
 }
 }  // namespace
 
+// Index of the smallest kept block for a buffer of `need` bytes, or -1.
+static int best_block(const std::vector<Block>& blocks, int device, size_t need, bool done) {
+    int best = -1;
+    for (size_t i = 0; i < blocks.size(); ++i) {
+        const Block& b = blocks[i];
+        if (b.device == device && b.done == done && b.cap >= need && b.cap <= block_for(need) &&
+            (best < 0 || b.cap < blocks[best].cap))
+            best = (int)i;
+    }
+    return best;
+}
+
+static Block take(std::vector<Block>& blocks, int i) {
+    const Block b = blocks[i];
+    blocks.erase(blocks.begin() + i);
+    return b;
+}
+
+bool dev_wait() noexcept {
+    void* p = nullptr;
+    if (hipMalloc(&p, 512) == hipSuccess && hipFree(p) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+static thread_local bool all_done = false;
+DoneScope::DoneScope(bool done) noexcept : before(all_done) { all_done = all_done || done; }
+DoneScope::~DoneScope() { all_done = before; }
+
+// Waits until the blocks of the current device that may still be in use are
+// idle.  They are out of other threads' reach meanwhile.
+static void settle(Idle& c, int device) {
+    std::vector<Block> busy;
+    {
+        std::lock_guard<std::mutex> guard(c.mu);
+        for (size_t i = 0; i < c.blocks.size();)
+            if (c.blocks[i].device == device && !c.blocks[i].done) busy.push_back(take(c.blocks, (int)i));
+            else ++i;
+    }
+    const bool waited = dev_wait();
+    std::lock_guard<std::mutex> guard(c.mu);
+    for (Block& b : busy) {
+        b.done = waited;
+        c.blocks.push_back(b);
+    }
+}
+
 void* dev_acquire(size_t n, size_t& cap, int& device) {
     MSR_HIP(hipGetDevice(&device));
     cap = (n + 511) / 512 * 512;
@@ -81,19 +131,18 @@ void* dev_acquire(size_t n, size_t& cap, int& device) {
         cap = SIZE_MAX / 4;  // more than any device has: fails below
     } else {
         Idle& c = idle();
-        std::lock_guard<std::mutex> guard(c.mu);
-        size_t best = c.blocks.size();
-        for (size_t i = 0; i < c.blocks.size(); ++i) {
-            const Block& b = c.blocks[i];
-            if (b.device == device && b.cap >= cap && b.cap <= block_for(cap) &&
-                (best == c.blocks.size() || b.cap < c.blocks[best].cap))
-                best = i;
+        std::unique_lock<std::mutex> guard(c.mu);
+        int i = best_block(c.blocks, device, cap, true);
+        if (i < 0 && best_block(c.blocks, device, cap, false) >= 0) {
+            guard.unlock();
+            settle(c, device);
+            guard.lock();
+            i = best_block(c.blocks, device, cap, true);
         }
-        if (best < c.blocks.size()) {
-            void* p = c.blocks[best].p;
-            cap = c.blocks[best].cap;
-            c.blocks.erase(c.blocks.begin() + best);
-            return p;
+        if (i >= 0) {
+            const Block b = take(c.blocks, i);
+            cap = b.cap;
+            return b.p;
         }
     }
     void* p = nullptr;
@@ -105,10 +154,9 @@ void* dev_acquire(size_t n, size_t& cap, int& device) {
     return p;
 }
 
-void dev_release(void* p, size_t cap, int device) noexcept {
+void dev_release(void* p, size_t cap, int device, bool done) noexcept {
     OnDevice on(device);
-    // not idle (or not known to be): hipFree waits by itself
-    if (!on.ok || !may_stay(cap) || hipDeviceSynchronize() != hipSuccess) {
+    if (!on.ok || !may_stay(cap)) {  // hipFree waits by itself
         (void)hipGetLastError();
         (void)hipFree(p);
         return;
@@ -117,7 +165,7 @@ void dev_release(void* p, size_t cap, int device) noexcept {
     try {
         Idle& c = idle();
         std::lock_guard<std::mutex> guard(c.mu);
-        c.blocks.push_back({p, cap, device});
+        c.blocks.push_back({p, cap, device, done || all_done});
         p = nullptr;
         size_t bytes = 0, count = 0;
         for (const Block& b : c.blocks)

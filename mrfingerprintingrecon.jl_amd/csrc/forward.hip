@@ -231,7 +231,7 @@ static const FwdPlan& fwd_plan(const msr_traj* traj, const FwdGeom& g, hipStream
     const int M = (int)traj->M;
     p->nry = (int)ceil_div(g.n[1], FW_TY);
     const int nr = (int)ceil_div(g.n[0], FW_TX) * p->nry;
-    DevBuf keys, sorted, idx, temp, first, nb, pos;
+    TempBuf keys{st}, sorted{st}, idx{st}, temp{st}, first{st}, nb{st}, pos{st};
     keys.alloc(sizeof(int) * M);
     sorted.alloc(sizeof(int) * M);
     idx.alloc(sizeof(int) * M);
@@ -413,7 +413,7 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
     const size_t ab = plan ? (sizeof(float2) * (size_t)nch * nos[0] * NN[1] + 255) / 256 * 256
                            : sizeof(float2) * (size_t)nch * Gos;
     const size_t bb = plan ? sizeof(float2) * (size_t)K * CB * PLANE_COIL_GROUP * Gos : ab;
-    DevBuf work;
+    TempBuf work{st};
     work.alloc(mb + zb + ab + bb);
     float2* mp = maps ? work.as<float2>() : nullptr;
     float2* Z = reinterpret_cast<float2*>(work.as<char>() + mb);

@@ -38,8 +38,21 @@ namespace msr {
 // Device memory behind DevBuf (devbuf.hip): blocks of freed buffers are kept,
 // up to a bounded number of idle bytes per device, and handed out again.
 void* dev_acquire(size_t n, size_t& cap, int& device);
-// Waits for the device (as hipFree does), then keeps or frees the block.
-void dev_release(void* p, size_t cap, int device) noexcept;
+// Keeps or frees the block; done: nothing queued on the device uses it any more
+// (else it is handed out only after the device has been waited for).
+void dev_release(void* p, size_t cap, int device, bool done) noexcept;
+// Waits for everything queued on the current device, by a hipFree, which does:
+// hipDeviceSynchronize is refused while any thread captures a stream, and ends
+// that capture.  False if that failed.
+bool dev_wait() noexcept;
+// While one with done set lives on a thread, nothing queued uses what the thread
+// releases.
+struct DoneScope {
+    bool before;
+    explicit DoneScope(bool done) noexcept;
+    ~DoneScope();
+    DoneScope(const DoneScope&) = delete;
+};
 // Frees the idle blocks of the device; their bytes.
 size_t dev_trim(int device) noexcept;
 
@@ -53,8 +66,8 @@ struct DevBuf {
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { release(); }
-    void release() {
-        if (p) dev_release(p, cap, device);  // in-flight kernels may still use p
+    void release(bool done = false) {  // not done: in-flight kernels may still use p
+        if (p) dev_release(p, cap, device, done);
         p = nullptr;
         bytes = cap = 0;
     }
@@ -66,6 +79,19 @@ struct DevBuf {
         bytes = n;
     }
     template <class T> T* as() const { return reinterpret_cast<T*>(p); }
+};
+
+// Temporary of a function that works on one stream: waits for it at the end, so
+// that the block is idle at once.
+struct TempBuf : DevBuf {
+    hipStream_t stream;
+    explicit TempBuf(hipStream_t st) : stream(st) {}
+    ~TempBuf() {
+        if (!p) return;
+        const bool done = hipStreamSynchronize(stream) == hipSuccess;
+        if (!done) (void)hipGetLastError();
+        release(done);
+    }
 };
 
 const float2* twiddle_table(msr_ctx* ctx, int n);

@@ -130,7 +130,7 @@ __global__ __launch_bounds__(HASH_THREADS) void hash_kernel(const uint32_t* __re
 // Hashes of nbuf device buffers (one partial-sum launch each, one read-back).
 static void hash_device(const void* const* bufs, const uint64_t* nbytes, int nbuf, uint64_t seed,
                         hipStream_t st, uint64_t (*out)[2]) {
-    DevBuf part;
+    TempBuf part{st};
     part.alloc(sizeof(uint64_t) * 2 * HASH_BLOCKS * nbuf);
     std::vector<int> blocks(nbuf);
     for (int b = 0; b < nbuf; ++b) {
@@ -218,7 +218,7 @@ void kernel_save(const msr_normalop* op, const char* path, const uint64_t* key, 
     const size_t kb = sizeof(int64_t) * (size_t)op->nkm, lb = es * (size_t)op->P * op->nkm;
     std::vector<uint8_t> payload(kb + lb);
     if (op->nkm > 0) {
-        DevBuf dl, dk;
+        TempBuf dl{st}, dk{st};
         dl.alloc(lb);
         dk.alloc(kb);
         op_export(op, dl.p, dk.as<int64_t>(), st);
@@ -341,7 +341,7 @@ msr_normalop* kernel_load(msr_ctx* ctx, const char* path, const uint64_t* expect
                     (unsigned long long)h.key[0], (unsigned long long)h.key[1]);
     std::unique_ptr<msr_normalop> op(op_new(ctx, (int)h.d, h.N, (int)h.K, (int)h.lambda_real));
     op_set_cmaps(op.get(), ncoils, cmaps, st);
-    DevBuf dev;
+    TempBuf dev{st};
     dev.alloc(std::max<size_t>(payload.size(), 8));
     if (!payload.empty())
         MSR_HIP(hipMemcpyAsync(dev.p, payload.data(), payload.size(), hipMemcpyHostToDevice, st));

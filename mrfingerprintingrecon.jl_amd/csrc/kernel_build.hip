@@ -141,7 +141,7 @@ void build_kmask(const msr_traj* traj, const int64_t* n2, DevBuf& mask, DevBuf& 
         // tail bytes (grid sizes here are even, G is a multiple of 4)
         fail(MSR_ERR_UNSUPPORTED, "grid size not a multiple of 4");
     }
-    DevBuf other;
+    TempBuf other{st};
     other.alloc(G);
     uint8_t* cur = (d == 2 ? mask : other).as<uint8_t>();  // the last widening ends in mask
     fill_floats(cur, G / 4, 0.f, st);
@@ -157,7 +157,7 @@ void build_kmask(const msr_traj* traj, const int64_t* n2, DevBuf& mask, DevBuf& 
         cur = next;
     }
     const int64_t nb = ceil_div(G, 1024);
-    DevBuf counts, offs;
+    TempBuf counts{st}, offs{st};
     counts.alloc(sizeof(int) * nb);
     offs.alloc(sizeof(int64_t) * (nb + 1));
     hipLaunchKernelGGL(mask_count_kernel, dim3((unsigned)nb), dim3(1024), 0, st,
@@ -194,7 +194,7 @@ void op_build_from_traj(msr_normalop* op, const msr_traj* traj, const void* U, i
         G4 *= n4[a];
     }
     // kmask
-    DevBuf mask;
+    TempBuf mask{st};
     build_kmask(traj, n2, mask, *op->kmask, op->nkm, st);
 
     // pair tables (packed order)
@@ -205,7 +205,7 @@ void op_build_from_traj(msr_normalop* op, const msr_traj* traj, const void* U, i
             pj[p] = j;
             pk[p] = k;
         }
-    DevBuf pairs;
+    TempBuf pairs{st};
     pairs.alloc(sizeof(int) * 2 * P);
     MSR_HIP(hipMemcpyAsync(pairs.p, pj.data(), sizeof(int) * P, hipMemcpyHostToDevice, st));
     MSR_HIP(hipMemcpyAsync(pairs.as<int>() + P, pk.data(), sizeof(int) * P, hipMemcpyHostToDevice, st));
@@ -229,7 +229,7 @@ void op_build_from_traj(msr_normalop* op, const msr_traj* traj, const void* U, i
     // MSR_KERNEL_TILES=1)
     const char* tiled = getenv("MSR_KERNEL_TILES");
     bool gather = kernel_spread_supported(d, n4) && !(tiled && atoi(tiled));
-    KernelSpread ks;
+    KernelSpread ks(st);
     const SpreadPlan* plan = nullptr;
     // Pairs per chunk: as many as the budget holds, less what would begin a
     // row tile of the gather, whose cost is by the tile (16 real or 8 complex
@@ -239,7 +239,7 @@ void op_build_from_traj(msr_normalop* op, const msr_traj* traj, const void* U, i
     // The gather's tables come on top, 64 d + 16 bytes per sample; where they do
     // not fit, the tiles do without.
     int pc = 0;
-    DevBuf A, B;
+    TempBuf A{st}, B{st};
     auto slab = [&](int nch) { return gather ? 0 : spread_workspace_bytes(*plan, nch, f64); };
     auto prepare = [&](size_t budget) {
         if (gather) ks.build(traj, n4, st);

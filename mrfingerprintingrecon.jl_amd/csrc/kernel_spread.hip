@@ -252,7 +252,7 @@ void KernelSpread::build(const msr_traj* traj, const int64_t* grid_n, hipStream_
     }
     MSR_REQUIRE(nbins < (int64_t)INT32_MAX, MSR_ERR_UNSUPPORTED, "grid too large");
     const KernelGeom g = geom_of(*this);
-    DevBuf keys, sorted, idx, perm, temp;
+    TempBuf keys{st}, sorted{st}, idx{st}, perm{st}, temp{st};
     keys.alloc(sizeof(int) * M);
     sorted.alloc(sizeof(int) * M);
     idx.alloc(sizeof(int) * M);

@@ -13,11 +13,12 @@ struct KernelSpread {
     int d = 2;
     int n[3] = {1, 1, 1}, nb[3] = {1, 1, 1};
     int64_t M = 0;
-    DevBuf cells;   // (M) int4: floor cell per dimension, frame
-    DevBuf wts;     // (M, d, 8) double: ES weights of the cells c - 3 .. c + 4
-    DevBuf first;   // (bins + 1) int32: first sorted sample of a bin
-    DevBuf vals;    // pair products per frame (basis values only)
+    TempBuf cells;  // (M) int4: floor cell per dimension, frame
+    TempBuf wts;    // (M, d, 8) double: ES weights of the cells c - 3 .. c + 4
+    TempBuf first;  // (bins + 1) int32: first sorted sample of a bin
+    TempBuf vals;   // pair products per frame (basis values only)
     bool built = false;
+    explicit KernelSpread(hipStream_t st) : cells(st), wts(st), first(st), vals(st) {}
     // Once; again does nothing, unless an allocation failed.
     void build(const msr_traj* traj, const int64_t* grid, hipStream_t st);
     void release();  // the tables

@@ -265,7 +265,7 @@ void op_load_packed(msr_normalop* op, const void* lambda, const int64_t* kmask, 
     op->kmask->alloc(sizeof(int64_t) * std::max<int64_t>(nkm, 1));
     if (nkm > 0)
         MSR_HIP(hipMemcpyAsync(op->kmask->p, kmask, sizeof(int64_t) * nkm, hipMemcpyDeviceToDevice, st));
-    DevBuf bad;
+    TempBuf bad{st};
     bad.alloc(sizeof(int));
     fill_floats(bad.p, 1, 0.f, st);
     if (nkm > 0) {

@@ -120,7 +120,7 @@ const SpreadPlan& spread_plan(const msr_traj* traj, const int64_t* n, hipStream_
         g.nb[a] = p->nb[a];
     }
     const int M = (int)traj->M;
-    DevBuf binid, binsorted, idx, temp;
+    TempBuf binid{st}, binsorted{st}, idx{st}, temp{st};
     binid.alloc(sizeof(int) * M);
     binsorted.alloc(sizeof(int) * M);
     idx.alloc(sizeof(int) * M);
@@ -446,7 +446,7 @@ static void spread_t(const msr_traj* traj, const SpreadPlan& plan, const ValueSr
                                traj->kc.as<float>(), traj->frame.as<int>(), plan.perm.as<int>(),
                                plan.offs.as<int>(), g, src, nch, 0, (AT*)nullptr, grid);
         } else {
-            DevBuf work;
+            TempBuf work{st};
             work.alloc(per_ch * cpp);
             for (int c0 = 0; c0 < nch; c0 += cpp) {
                 const int nc = std::min(cpp, nch - c0);

@@ -150,13 +150,13 @@ void spread_streams(const msr_traj* traj, SpreadPlan& plan, hipStream_t st) {
     }
     const int64_t ntiles = (int64_t)g.nb[0] * g.nb[1];
     const int64_t Mp = std::max<int64_t>(M, 1);
-    DevBuf frac;
+    TempBuf frac{st};
     frac.alloc(sizeof(float2) * Mp);
     plan.cell.alloc(sizeof(int2) * Mp);
     plan.frame_s.alloc(sizeof(int) * Mp);
     plan.jsel_s.alloc(sizeof(int64_t) * Mp);
     plan.kc_s.alloc(sizeof(float2) * Mp);
-    DevBuf npp, ppos, keys, keys_sorted, vals, temp, first;
+    TempBuf npp{st}, ppos{st}, keys{st}, keys_sorted{st}, vals{st}, temp{st}, first{st};
     npp.alloc(sizeof(int) * (Mp + 1));
     ppos.alloc(sizeof(int) * (Mp + 1));
     const int grid = (int)std::min<int64_t>((M + 255) / 256, 8192);

@@ -168,13 +168,13 @@ void spread_streams3(const msr_traj* traj, SpreadPlan& plan, hipStream_t st) {
     const int64_t nblocks = (int64_t)g.nb[0] * g.nb[1] * g.nb[2];
     MSR_REQUIRE(nblocks < ((int64_t)1 << 30), MSR_ERR_UNSUPPORTED, "grid too large");
     const int64_t Mp = std::max<int64_t>(M, 1);
-    DevBuf frac;
+    TempBuf frac{st};
     frac.alloc(sizeof(float4) * Mp);
     plan.cell.alloc(sizeof(int4) * Mp);
     plan.frame_s.alloc(sizeof(int) * Mp);
     plan.jsel_s.alloc(sizeof(int64_t) * Mp);
     plan.r2_s.alloc(sizeof(float) * Mp);
-    DevBuf npp, ppos, keys, keys_sorted, vals, temp, first;
+    TempBuf npp{st}, ppos{st}, keys{st}, keys_sorted{st}, vals{st}, temp{st}, first{st};
     npp.alloc(sizeof(int) * (Mp + 1));
     ppos.alloc(sizeof(int) * (Mp + 1));
     const int grid = (int)std::min<int64_t>((M + 255) / 256, 8192);

@@ -192,7 +192,7 @@ msr_traj* traj_create(msr_ctx* ctx, int d, int64_t nsamp, int64_t nt, const floa
         MSR_CHECK_LAUNCH();
         return tj.release();
     }
-    DevBuf counts, offsets;
+    TempBuf counts{st}, offsets{st};
     counts.alloc(sizeof(int64_t) * nt);
     offsets.alloc(sizeof(int64_t) * nt);
     hipLaunchKernelGGL(count_frames_kernel, dim3(nt), dim3(256), 0, st, mask, nsamp,

@@ -73,7 +73,7 @@ void op_tune(msr_normalop* op, int am, int nrep, double* times, int* chosen, hip
     op_ensure_scratch(op, f64);
     const size_t es = f64 ? sizeof(double2) : sizeof(float2);
     const int64_t n = (int64_t)op->K * op->V;
-    DevBuf b, ref, ndiff;
+    TempBuf b{st}, ref{st}, ndiff{st};
     b.alloc(es * (size_t)n);
     ref.alloc(op->partial.bytes);
     ndiff.alloc(sizeof(int));

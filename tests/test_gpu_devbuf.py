@@ -1,6 +1,7 @@
 """Device memory kept for the library's next buffers: bounded, given back on
 request, and nothing large kept while the device is nearly full."""
 import gc
+import threading
 
 import numpy as np
 import pytest
@@ -96,3 +97,75 @@ def test_an_operator_takes_what_its_footprint_says(torch, msr):
     used = available(torch) - with_op
     print(f"used {used / 2**20:.1f} MiB, footprint {(own + kernel_bytes) / 2**20:.1f} MiB", flush=True)
     assert used <= (own + kernel_bytes) * 65 / 64 + (1 << 20)
+
+
+def test_allocations_beside_a_capture(torch, msr):
+    """One thread captures CG graphs of new operators while another constructs and
+    destroys operators: neither fails, and the solves keep their bits."""
+    rng = np.random.default_rng(3)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+    def protocol(n, k, nt, ns):
+        return n, dev(rng.uniform(-0.5, 0.5, size=(nt, ns, len(n))).astype(np.float32)), \
+            dev(rng.normal(size=(k, nt)).astype(np.float32))
+
+    solve, build = protocol((32, 24), 2, 8, 200), protocol((16, 16, 12), 2, 8, 300)
+    b = torch.randn(2 * 32 * 24, dtype=torch.complex64, device="cuda")
+
+    def solved():
+        return msr.cg(msr.NFFTNormalOp(*solve), b, maxiter=20, reltol=0.0, mode="graph")
+
+    want = solved()
+    msr.NFFTNormalOp(*build)      # tables
+    torch.cuda.synchronize()
+    failures, stop = [], threading.Event()
+
+    def guarded(body):
+        st = torch.cuda.Stream()
+        try:
+            with torch.cuda.stream(st):
+                body(st)
+        except Exception as e:
+            failures.append(repr(e))
+
+    def solver(st):
+        try:
+            for _ in range(150):
+                x = solved()
+                st.synchronize()
+                if not torch.equal(x, want):
+                    failures.append("bits")
+        finally:
+            stop.set()
+
+    def builder(st):
+        while not stop.is_set():
+            msr.NFFTNormalOp(*build)
+
+    threads = [threading.Thread(target=guarded, args=(f,)) for f in (solver, builder)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures[:3]
+
+
+def test_destroying_a_handle_waits_for_the_device(torch, msr):
+    """Its buffers go to the next caller, so work queued on any stream (here 30
+    matrix products, some milliseconds) has ended when a handle is gone."""
+    trj = torch.zeros((2, 50, 2), dtype=torch.float32, device="cuda")
+    a = torch.randn(4096, 4096, device="cuda")
+    a @ a
+    traj = msr.plan_trajectory(trj)
+    torch.cuda.synchronize()
+    st = torch.cuda.Stream()
+    done = torch.cuda.Event()
+    with torch.cuda.stream(st):
+        for _ in range(30):
+            b = a @ a
+        done.record(st)
+    running = not done.query()
+    del traj
+    gc.collect()
+    assert running and done.query()
+    del b
