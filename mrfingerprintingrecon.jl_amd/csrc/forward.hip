@@ -365,6 +365,8 @@ static bool fwd_batches_pay(int64_t nbatch, int64_t M, int C) {
     return 8 * nbatch * ceil_div(C, 8) <= 5 * M * ceil_div(C, 4);
 }
 
+constexpr size_t FW_WORK = (size_t)6 << 30;  // grids of a chunk of coils (interp_kernel)
+
 // Device copy of the coil maps, packed (C, V): one launch per 32 coils.
 constexpr int FW_MAPS = 32;
 struct FwdMaps {
@@ -395,7 +397,6 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
         V *= N[a];
         Gos *= nos[a];
     }
-    const int nch = C * K;
     const FwdGeom g{{nos[0], nos[1], nos[2]}};
     const FwdPlan* plan = nullptr;
     if (d == 2 && U && fwd_batches_possible(traj, nos, C)) {
@@ -408,10 +409,15 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
     // workspace: coil maps, then S_c x_k and two grid buffers, or (matrix
     // cores) the row transforms and the grid in groups of 8 coils.  The call's
     // own, from the idle blocks: calls on one trajectory run side by side, and
-    // nothing stays with the handle (128 x 128 x 128, 16 coils, K = 4: 18 GB)
-    const size_t zb = plan ? 0 : sizeof(float2) * (size_t)nch * V;
-    const size_t ab = plan ? (sizeof(float2) * (size_t)nch * nos[0] * NN[1] + 255) / 256 * 256
-                           : sizeof(float2) * (size_t)nch * Gos;
+    // nothing stays with the handle.  One wavefront per sample takes a multiple of
+    // its groups' coils at a time, within FW_WORK bytes of grids, which the idle
+    // blocks can hold (128 x 128 x 128, 16 coils, K = 4: 18 GB at once, mapped for
+    // every call, took 20.3 ms, 4.6 GB in four chunks 19.6)
+    const size_t coil = sizeof(float2) * (size_t)K * (V + 2 * Gos);
+    const int Cw = plan ? C : (int)std::min<int64_t>(C, std::max<int64_t>(1, FW_WORK / coil / FW_CB) * FW_CB);
+    const size_t zb = plan ? 0 : sizeof(float2) * (size_t)Cw * K * V;
+    const size_t ab = plan ? (sizeof(float2) * (size_t)C * K * nos[0] * NN[1] + 255) / 256 * 256
+                           : sizeof(float2) * (size_t)Cw * K * Gos;
     const size_t bb = plan ? sizeof(float2) * (size_t)K * CB * PLANE_COIL_GROUP * Gos : ab;
     TempBuf work{st};
     work.alloc(mb + zb + ab + bb);
@@ -462,75 +468,80 @@ void forward_model(msr_ctx* ctx, const msr_traj* traj, int d, const int64_t* N, 
         MSR_HIP(hipStreamSynchronize(st));  // the workspace is freed on return
         return;
     }
-    int grid = (int)std::min<int64_t>(((int64_t)nch * V + 255) / 256, 16384);
-    hipLaunchKernelGGL(expand_kernel, dim3(grid), dim3(256), 0, st, (const float2*)x, mp, C, K, V, Z);
-    MSR_CHECK_LAUNCH();
-    // x: centred placement + deapodisation, forward FFT over 2Nx  -> A [ch][z][y][qx]
-    LinePass px;
-    px.in = Z;
-    px.out = A;
-    px.nf = (int)nos[0];
-    px.dir = -1;
-    px.lin = (int)NN[0];
-    px.isel = SEL_CENTER;
-    px.win = deapod_table(ctx, (int)nos[0], (int)NN[0], SEL_CENTER);
-    px.lout = (int)nos[0];
-    px.sel = SEL_FIRST;
-    px.nlines = (int64_t)nch * NN[1] * NN[2];
-    px.in_pitch = NN[0];
-    px.out_pitch = nos[0];
-    run_rows(px, ctx, st);
-    // y: A [ch][z][y][qx] -> B [ch][z][qy][qx]
-    LinePass py;
-    py.in = A;
-    py.out = B;
-    py.nf = (int)nos[1];
-    py.dir = -1;
-    py.lin = (int)NN[1];
-    py.isel = SEL_CENTER;
-    py.win = deapod_table(ctx, (int)nos[1], (int)NN[1], SEL_CENTER);
-    py.lout = (int)nos[1];
-    py.sel = SEL_FIRST;
-    py.nb = (int64_t)nch * NN[2];
-    py.ncols = nos[0];
-    py.in_bstride = NN[1] * nos[0];
-    py.in_stride = nos[0];
-    py.out_bstride = nos[1] * nos[0];
-    py.out_stride = nos[0];
-    run_cols(py, ctx, st);
-    const float2* Gfin = B;
-    if (d == 3) {
-        // z: B [ch][z][qy][qx] -> A [ch][qz][qy][qx]
-        LinePass pz;
-        pz.in = B;
-        pz.out = A;
-        pz.nf = (int)nos[2];
-        pz.dir = -1;
-        pz.lin = (int)NN[2];
-        pz.isel = SEL_CENTER;
-        pz.win = deapod_table(ctx, (int)nos[2], (int)NN[2], SEL_CENTER);
-        pz.lout = (int)nos[2];
-        pz.sel = SEL_FIRST;
-        pz.nb = nch;
-        pz.ncols = nos[1] * nos[0];
-        pz.in_bstride = NN[2] * nos[1] * nos[0];
-        pz.in_stride = nos[1] * nos[0];
-        pz.out_bstride = Gos;
-        pz.out_stride = nos[1] * nos[0];
-        run_cols(pz, ctx, st);
-        Gfin = A;
+    for (int c0 = 0; c0 < C; c0 += Cw) {
+        const int nc = std::min(Cw, C - c0), nch = nc * K;
+        float2* o = (float2*)out + (int64_t)c0 * nsel;
+        int grid = (int)std::min<int64_t>(((int64_t)nch * V + 255) / 256, 16384);
+        hipLaunchKernelGGL(expand_kernel, dim3(grid), dim3(256), 0, st, (const float2*)x,
+                           mp ? mp + (int64_t)c0 * V : nullptr, nc, K, V, Z);
+        MSR_CHECK_LAUNCH();
+        // x: centred placement + deapodisation, forward FFT over 2Nx  -> A [ch][z][y][qx]
+        LinePass px;
+        px.in = Z;
+        px.out = A;
+        px.nf = (int)nos[0];
+        px.dir = -1;
+        px.lin = (int)NN[0];
+        px.isel = SEL_CENTER;
+        px.win = deapod_table(ctx, (int)nos[0], (int)NN[0], SEL_CENTER);
+        px.lout = (int)nos[0];
+        px.sel = SEL_FIRST;
+        px.nlines = (int64_t)nch * NN[1] * NN[2];
+        px.in_pitch = NN[0];
+        px.out_pitch = nos[0];
+        run_rows(px, ctx, st);
+        // y: A [ch][z][y][qx] -> B [ch][z][qy][qx]
+        LinePass py;
+        py.in = A;
+        py.out = B;
+        py.nf = (int)nos[1];
+        py.dir = -1;
+        py.lin = (int)NN[1];
+        py.isel = SEL_CENTER;
+        py.win = deapod_table(ctx, (int)nos[1], (int)NN[1], SEL_CENTER);
+        py.lout = (int)nos[1];
+        py.sel = SEL_FIRST;
+        py.nb = (int64_t)nch * NN[2];
+        py.ncols = nos[0];
+        py.in_bstride = NN[1] * nos[0];
+        py.in_stride = nos[0];
+        py.out_bstride = nos[1] * nos[0];
+        py.out_stride = nos[0];
+        run_cols(py, ctx, st);
+        const float2* Gfin = B;
+        if (d == 3) {
+            // z: B [ch][z][qy][qx] -> A [ch][qz][qy][qx]
+            LinePass pz;
+            pz.in = B;
+            pz.out = A;
+            pz.nf = (int)nos[2];
+            pz.dir = -1;
+            pz.lin = (int)NN[2];
+            pz.isel = SEL_CENTER;
+            pz.win = deapod_table(ctx, (int)nos[2], (int)NN[2], SEL_CENTER);
+            pz.lout = (int)nos[2];
+            pz.sel = SEL_FIRST;
+            pz.nb = nch;
+            pz.ncols = nos[1] * nos[0];
+            pz.in_bstride = NN[2] * nos[1] * nos[0];
+            pz.in_stride = nos[1] * nos[0];
+            pz.out_bstride = Gos;
+            pz.out_stride = nos[1] * nos[0];
+            run_cols(pz, ctx, st);
+            Gfin = A;
+        }
+        const int64_t waves = traj->M;
+        const int blocks = (int)std::min<int64_t>((waves * 64 + 255) / 256, 65536);
+        if (d == 2)
+            hipLaunchKernelGGL(interp_kernel<2>, dim3(blocks), dim3(256), 0, st, traj->kc.as<float>(),
+                               traj->frame.as<int>(), traj->sel.p ? traj->sel.as<int64_t>() : nullptr,
+                               traj->M, nsel, Gfin, g, K, nc, U, u_real, traj->nt, o);
+        else
+            hipLaunchKernelGGL(interp_kernel<3>, dim3(blocks), dim3(256), 0, st, traj->kc.as<float>(),
+                               traj->frame.as<int>(), traj->sel.p ? traj->sel.as<int64_t>() : nullptr,
+                               traj->M, nsel, Gfin, g, K, nc, U, u_real, traj->nt, o);
+        MSR_CHECK_LAUNCH();
     }
-    const int64_t waves = traj->M;
-    const int blocks = (int)std::min<int64_t>((waves * 64 + 255) / 256, 65536);
-    if (d == 2)
-        hipLaunchKernelGGL(interp_kernel<2>, dim3(blocks), dim3(256), 0, st, traj->kc.as<float>(),
-                           traj->frame.as<int>(), traj->sel.p ? traj->sel.as<int64_t>() : nullptr,
-                           traj->M, nsel, Gfin, g, K, C, U, u_real, traj->nt, (float2*)out);
-    else
-        hipLaunchKernelGGL(interp_kernel<3>, dim3(blocks), dim3(256), 0, st, traj->kc.as<float>(),
-                           traj->frame.as<int>(), traj->sel.p ? traj->sel.as<int64_t>() : nullptr,
-                           traj->M, nsel, Gfin, g, K, C, U, u_real, traj->nt, (float2*)out);
-    MSR_CHECK_LAUNCH();
     MSR_HIP(hipStreamSynchronize(st));  // the workspace is freed on return
 }
 

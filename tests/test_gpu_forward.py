@@ -118,6 +118,16 @@ def test_workspace_goes_back(torch, msr, N, K, C):
     assert left < 32 << 20
 
 
+def test_coils_in_chunks(torch, msr):
+    """128 x 128 x 128, K = 4: the grids of nine coils exceed the workspace's bound,
+    so the coils go four at a time; the bits of three calls with those coils."""
+    x, trj, cm, U = problem(torch, (128, 128, 128), 4, 9, 4, 500)
+    traj = msr.plan_trajectory(trj)
+    y = msr.forward(x, traj, cmaps=cm, U=U)
+    for c in range(0, 9, 4):
+        assert torch.equal(y[c:c + 4], msr.forward(x, traj, cmaps=cm[c:c + 4], U=U))
+
+
 def test_few_coils_make_no_plan(torch, msr):
     """Three coils never take the matrix cores: 4 million samples are not sorted for
     them, and no sorted list (16 MB, and the batches) stays with the trajectory."""
