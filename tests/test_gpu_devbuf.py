@@ -66,7 +66,10 @@ def test_nothing_large_stays_while_the_device_is_nearly_full(torch, msr):
     rest = total // 16
     if free < rest:
         pytest.skip("device in use")
-    hold = torch.empty(free - rest, dtype=torch.uint8, device="cuda")
+    try:
+        hold = torch.empty(free - rest, dtype=torch.uint8, device="cuda")
+    except torch.cuda.OutOfMemoryError:
+        pytest.skip("device in use")
     try:
         assert torch.equal(first, kernel(torch, msr))
         freed = msr.trim()
@@ -151,8 +154,8 @@ def test_allocations_beside_a_capture(torch, msr):
 
 
 def test_destroying_a_handle_waits_for_the_device(torch, msr):
-    """Its buffers go to the next caller, so work queued on any stream (here 30
-    matrix products, some milliseconds) has ended when a handle is gone."""
+    """Its buffers go to the next caller, so work queued on any stream (here 100
+    matrix products, about 100 ms) has ended when a handle is gone."""
     trj = torch.zeros((2, 50, 2), dtype=torch.float32, device="cuda")
     a = torch.randn(4096, 4096, device="cuda")
     a @ a
@@ -161,7 +164,7 @@ def test_destroying_a_handle_waits_for_the_device(torch, msr):
     st = torch.cuda.Stream()
     done = torch.cuda.Event()
     with torch.cuda.stream(st):
-        for _ in range(30):
+        for _ in range(100):
             b = a @ a
         done.record(st)
     running = not done.query()
